@@ -106,9 +106,9 @@ CONNECTOR_PROFILE = {
 
 
 def hip_kernel_names(codec, S: int, H: int, D: int, bits: int, cplan=None) -> dict:
-    """Name of the HIP kernel each entry point runs for this geometry (MFMA unless the
-    register-FWHT kernels are forced, quad-per-row or generic rows, or the geometry is
-    not MFMA-eligible)."""
+    """Name of the HIP kernel each entry point runs for this geometry (MFMA, wave tiles for
+    what those do not take, or the register-FWHT kernels: quad-per-row or generic rows
+    where they are forced or nothing else serves the geometry)."""
     default_axes = tuple(getattr(codec, "axes", ("channel", "token"))) == ("channel", "token")
     pow2 = D in (64, 128) and default_axes
     if D == 256 and H <= 16 and default_axes and codec.fwht == "mfma" and codec.transform:
@@ -134,12 +134,20 @@ def hip_kernel_names(codec, S: int, H: int, D: int, bits: int, cplan=None) -> di
         if cplan is not None and getattr(cplan, "workspace", None) is not None:  # the one-pass kernel runs
             names["kvmi_compress_paged"] = f"onepass_kernel<{D // 32}, {bits}, false>"
         return names
-    if pow2 and H <= 16 and 128 % H == 0 and codec.fwht != "rows":  # quad-per-row register FWHT
+    if codec.fwht == "valu" and pow2 and H <= 16 and 128 % H == 0:  # quad-per-row register FWHT
         return {"kvmi_encode_paged": f"encode_kernel<{D}, {bits}>", "kvmi_decode_paged": f"decode_kernel<{D}, {bits}>",
                 "kvmi_kstats_paged": f"kstats_kernel<{D}>", "finalize": "kstats_finalize_kernel"}
     lpr = 1 << max(0, (D // 16 - 1).bit_length())  # generic rows: next_pow2(D / 16) lanes per row
-    return {"kvmi_encode_paged": f"rows_encode_kernel<{lpr}, {bits}>", "kvmi_decode_paged":
+    rows = {"kvmi_encode_paged": f"rows_encode_kernel<{lpr}, {bits}>", "kvmi_decode_paged":
             f"rows_decode_kernel<{lpr}, {bits}>", "kvmi_kstats_paged": f"rows_stats_kernel<{lpr}>",
+            "finalize": "rows_finalize_kernel"}
+    if codec.fwht != "mfma" or D not in (64, 80, 96, 112, 128, 160, 192, 224, 256) or H > 32:
+        return rows
+    tr = "true" if codec.transform else "false"  # wave tiles, where the workgroup's LDS allows (tile_eligible)
+    w = 4 if bits == 4 else 0
+    return {"kvmi_encode_paged": f"tile_encode_kernel<{D}, {tr}, {w}>",
+            "kvmi_decode_paged": f"tile_decode_kernel<{D}, {tr}, {w}>",
+            "kvmi_kstats_paged": f"tile_stats_kernel<{D}>" if codec.transform else "tile_plain_stats_kernel",
             "finalize": "rows_finalize_kernel"}
 
 

@@ -1,6 +1,8 @@
 // Fused paged compress / decompress kernels for gfx950, register FWHT, one quad of
-// lanes per row (D in {64, 128}, H dividing 128, H <= 16; other geometries run the
-// generic row kernels of kvmi_rows.hip, the transform profile mostly the MFMA kernels).
+// lanes per row (D in {64, 128}, H dividing 128, H <= 16), run where the caller forces
+// them (KVMI_F_VALU_FWHT), and the entry points of the paged codec: the transform profile
+// runs the MFMA kernels, what those do not take the wave tiles (kvmi_tile.hpp), the rest the
+// generic row kernels (kvmi_rows.hip); see the families in kvmi_common.hpp.
 //
 // Work unit: a workgroup of 512 threads (8 wave64s) owns a run of paged blocks of
 // one (request, layer) job.  The run's rows (one row = one token x one KV head =
@@ -426,6 +428,8 @@ extern "C" int kvmi_kstats_paged(const kvmi_geometry* geom, const kvmi_layer_job
   } else if (mfma_eligible(g)) {
     rc = mfma_kstats(g, jobs, num_jobs, max_blocks, err, st);
     if (rc) return rc;
+  } else if (tile_eligible(g, max_blocks)) {
+    return tile_kstats(g, jobs, num_jobs, max_blocks, err, st);  // statistics of both parts + their finalize
   } else if (!quad_eligible(g)) {
     return rows_kstats(g, jobs, num_jobs, max_blocks, err, st);  // statistics of both parts + their finalize
   } else {
@@ -457,6 +461,7 @@ extern "C" int kvmi_encode_paged(const kvmi_geometry* geom, const kvmi_layer_job
   Geo v;
   if (paired_view(g, &v)) return mfma_encode(v, jobs, num_jobs, max_blocks, err, st);
   if (mfma_eligible(g)) return mfma_encode(g, jobs, num_jobs, max_blocks, err, st);
+  if (tile_eligible(g, max_blocks)) return tile_encode(g, jobs, num_jobs, max_blocks, err, st);
   if (!quad_eligible(g)) return rows_encode(g, jobs, num_jobs, max_blocks, err, st);
   set_valu_bpw(&g);
   dim3 grid((unsigned)((max_blocks + g.bpw - 1) / g.bpw), (unsigned)num_jobs);
@@ -480,6 +485,7 @@ extern "C" int kvmi_decode_paged(const kvmi_geometry* geom, const kvmi_layer_job
   Geo v;
   if (paired_view(g, &v)) return mfma_decode(v, jobs, num_jobs, max_blocks, err, st);
   if (mfma_eligible(g)) return mfma_decode(g, jobs, num_jobs, max_blocks, err, st);
+  if (tile_eligible(g, max_blocks) && tile_decodes(g)) return tile_decode(g, jobs, num_jobs, max_blocks, err, st);
   if (!quad_eligible(g)) return rows_decode(g, jobs, num_jobs, max_blocks, err, st);
   set_valu_bpw(&g);
   dim3 grid((unsigned)((max_blocks + g.bpw - 1) / g.bpw), (unsigned)num_jobs);

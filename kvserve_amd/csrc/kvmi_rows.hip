@@ -1,6 +1,7 @@
 // Generic-geometry paged compress / decompress kernels for gfx950 (register FWHT).
 //
-// They serve the geometries the MFMA and quad-per-row kernels do not: any H up to 64
+// They serve the geometries that neither the MFMA kernels nor the wave tiles
+// (kvmi_tile.hpp) take, and any call that forces them: any H up to 64
 // and any D that is a multiple of 16 up to 256, with H * next_pow2(D) <= 8192.  A D
 // that is not a power of two is transformed as the reference does it
 // (hadamard_func.py:50-103): split into descending power-of-two chunks, each chunk
@@ -843,6 +844,12 @@ int rows_hadamard(const void* in, void* out, int64_t rows, int32_t H, int32_t D,
   return hipGetLastError() == hipSuccess ? KVMI_OK : KVMI_ELAUNCH;
 }
 
+// Keys of every channel- or tensor-axis part -> metadata (also behind tile_kstats).
+int rows_finalize(const Geo& g, const kvmi_layer_job* jobs, int32_t num_jobs, hipStream_t st) {
+  hipLaunchKernelGGL(rows_finalize_kernel, dim3((unsigned)num_jobs), dim3(kRWG), 0, st, g, jobs);
+  return hipGetLastError() == hipSuccess ? KVMI_OK : KVMI_ELAUNCH;
+}
+
 int rows_kstats(const Geo& g0, const kvmi_layer_job* jobs, int32_t num_jobs, int32_t max_blocks, int32_t*,
                 hipStream_t st) {
   Geo g = g0;
@@ -857,8 +864,7 @@ int rows_kstats(const Geo& g0, const kvmi_layer_job* jobs, int32_t num_jobs, int
     default: launch_stats<16>(g, grid, jobs, st); break;
   }
   if (hipGetLastError() != hipSuccess) return KVMI_ELAUNCH;
-  hipLaunchKernelGGL(rows_finalize_kernel, dim3((unsigned)num_jobs), dim3(kRWG), 0, st, g, jobs);
-  return hipGetLastError() == hipSuccess ? KVMI_OK : KVMI_ELAUNCH;
+  return rows_finalize(g, jobs, num_jobs, st);
 }
 
 int rows_encode(const Geo& g0, const kvmi_layer_job* jobs, int32_t num_jobs, int32_t max_blocks, int32_t* err,

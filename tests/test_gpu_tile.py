@@ -1,0 +1,138 @@
+"""The wave-tile kernels (csrc/kvmi_tile*) against the generic row kernels on the same calls.
+
+`fwht="rows"` forces the row kernels, which the oracle pins bit for bit
+(tests/test_gpu_configs.py, tests/test_gpu_axes.py).  The transform on the matrix cores adds
+in another fp32 order, so a value may land on the other side of a bf16 rounding boundary:
+symbols one level apart on at most 1e-4 of the elements, decoded values one bf16 ulp apart
+on at most 1e-3 of them (the bars of tests/test_gpu_configs.py).  Without a transform both
+do the same arithmetic and have to agree bit for bit.
+"""
+
+import pytest
+import torch
+
+from kvserve_amd.engine import FusedKVCodec
+from kvserve_amd.profiles import section_profile, whole_layer_profile
+
+pytestmark = pytest.mark.gpu
+
+TOP = {1: 2, 2: 3, 3: 7, 4: 15, 5: 31, 6: 60, 7: 100, 8: 200}
+CT = ("channel", "token")
+CASES = [
+    # heads, head_dim, block, bits, layout, axes, transform, blocks
+    (6, 96, 16, 4, "permuted", CT, True, 9),          # 5 tokens a tile, straddling blocks; 64 + 32 channels
+    (6, 96, 16, 4, "native", CT, True, 40),
+    (5, 80, 16, 3, "permuted", CT, True, 7),          # 16-channel tail, 30-byte rows
+    (1, 112, 4, 7, "permuted", CT, True, 3),          # T limited by the block size
+    (32, 64, 1, 5, "permuted", CT, True, 17),         # one token a tile, one-token blocks
+    (7, 160, 3, 6, "native", CT, True, 5),            # block size not a power of two
+    (4, 224, 16, 8, "permuted", CT, True, 2),
+    (12, 192, 16, 4, "permuted", CT, True, 5),        # 24 of 32 rows
+    (3, 256, 8, 4, "permuted", CT, True, 6),
+    (8, 128, 16, 4, "permuted", ("token", "channel"), True, 33),
+    (8, 64, 16, 4, "permuted", ("tensor", "tensor"), True, 33),
+    (2, 80, 16, 2, "native", ("tensor", "token"), True, 1),
+    (10, 128, 16, 1, "permuted", ("channel", "channel"), True, 4),
+    (8, 128, 16, 4, "permuted", CT, False, 33),
+    (6, 96, 16, 8, "native", ("token", "token"), False, 9),
+    (16, 80, 2, 3, "permuted", ("tensor", "channel"), False, 9),
+]
+
+
+def _bits(t):
+    return t.view(torch.int16).to(torch.int32)
+
+
+def _unpack(stream, bits):
+    body = stream[16:].to(torch.int64)
+    at = torch.arange(body.numel() * 8 // bits, device=body.device) * bits
+    pad = torch.nn.functional.pad(body, (0, 2))
+    word = pad[at // 8] | (pad[at // 8 + 1] << 8)
+    return (word >> (at % 8)) & ((1 << bits) - 1)
+
+
+def _run(case, pools, ids, profiles, fwht):
+    H, D, S, bits, layout, axes, transform, _ = case
+    codec = FusedKVCodec(H, D, S, bits, 7, transform=transform, layout=layout, axes=axes, fwht=fwht)
+    plan = codec.plan_compress(pools, ids, profiles)
+    plan.packet.kmeta.zero_()
+    plan.packet.vmeta.zero_()
+    plan.run()
+    plan.run()  # the statistics keys are left ready for the next run
+    return codec, plan
+
+
+def _pools(case, gen, layers):
+    H, D, S, _, _, _, _, B = case
+    return [torch.randn((2, 2 * B + 3, S, H, D), generator=gen, device="cuda").to(torch.bfloat16) for _ in range(layers)]
+
+
+def _profiles(case, layers):
+    H, bits = case[0], case[3]
+    top, low = TOP[bits], max(2, TOP[bits] // 2)
+    mixed = section_profile([h % 3 == 1 for h in range(H)], top, top, low, low)
+    return [mixed if l % 2 == 0 else whole_layer_profile(H, top, low) for l in range(layers)]
+
+
+@pytest.mark.parametrize("case", CASES, ids=lambda c: "-".join(str(x) for x in c[:5]) + "-" + "".join(a[1] for a in c[5]) + ("" if c[6] else "-plain") + f"-{c[7]}")
+def test_tile_matches_rows(case):
+    H, D, S, bits, layout, axes, transform, B = case
+    layers = 2
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    pools = _pools(case, gen, layers)
+    order = torch.randperm(2 * B + 3, generator=torch.Generator().manual_seed(4)).tolist()
+    profiles = _profiles(case, layers)
+    tile, a = _run(case, pools, order[:B], profiles, "mfma")
+    rows, b = _run(case, pools, order[:B], profiles, "rows")
+    assert a.error_code() == b.error_code()
+    for x, y in zip(a.packet.streams, b.packet.streams):
+        if transform:
+            d = (_unpack(x, bits) - _unpack(y, bits)).abs()
+            assert int(d.max()) <= 1 and int((d > 0).sum()) <= 1e-4 * d.numel()
+        else:
+            assert torch.equal(x, y)
+    assert torch.equal(a.packet.kmeta, b.packet.kmeta) and torch.equal(a.packet.vmeta, b.packet.vmeta)
+    out = []
+    for codec in (tile, rows):
+        dst = [torch.full_like(p, 7.0) for p in pools]
+        plan = codec.plan_decompress(b.packet, dst, order[-B:])
+        plan.run()
+        assert plan.error_code() == b.error_code()
+        out.append(dst)
+    for x, y in zip(*out):
+        d = (_bits(x) - _bits(y)).abs()
+        if transform:
+            assert int(d.max()) <= 1 and int((d > 0).sum()) <= 1e-3 * d.numel()
+        else:
+            assert not d.any()
+
+
+@pytest.mark.parametrize("case", [c for c in CASES if c[7] >= 9], ids=lambda c: f"{c[0]}-{c[1]}-{c[3]}-{c[6]}")
+def test_tile_special_values(case):
+    """Zeros, constants, an infinity and a NaN in a row: the same symbols, metadata and caches
+    as the row kernels (a NaN takes the top level, statistics pass it over)."""
+    B, transform = case[7], case[6]
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    pools = _pools(case, gen, 1)
+    order = list(range(2 * B + 3))
+    pools[0][:, 0] = 0.0
+    pools[0][:, 1] = 1.5
+    pools[0][:, 2, 0, 0, 5] = float("inf")
+    pools[0][:, 3, 0, case[0] - 1, 8] = float("-inf")
+    pools[0][:, 4, 0, 0, 17] = float("nan")
+    profiles = _profiles(case, 1)
+    tile, a = _run(case, pools, order[:B], profiles, "mfma")
+    rows, b = _run(case, pools, order[:B], profiles, "rows")
+    assert a.error_code() == b.error_code()
+    same = lambda x, y: torch.equal(torch.nan_to_num(x.float(), nan=123.0), torch.nan_to_num(y.float(), nan=123.0))  # noqa: E731
+    assert same(a.packet.kmeta, b.packet.kmeta) and same(a.packet.vmeta, b.packet.vmeta)
+    d = (_unpack(a.packet.streams[0], case[3]) - _unpack(b.packet.streams[0], case[3])).abs()
+    assert int((d > 0).sum()) <= (1e-4 * d.numel() if transform else 0)
+    out = []
+    for codec in (tile, rows):
+        dst = [torch.zeros_like(p) for p in pools]
+        codec.plan_decompress(b.packet, dst, order[:B]).run()
+        out.append(dst[0])
+    x, y = (torch.nan_to_num(t.float(), nan=123.0, posinf=1e9, neginf=-1e9) for t in out)
+    close = (x - y).abs() <= (y.abs() * 2.0 ** -7 if transform else 0.0)
+    assert bool(close.all())
