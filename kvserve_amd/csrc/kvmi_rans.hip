@@ -20,9 +20,19 @@
 //   rans_compact_kernel  copies each block from its slot (or the raw input) to its
 //                        offset in the stream
 //   rans_decode_kernel   table -> decode (steps 0..255) -> packed symbols
-// Division x / f by the 12-bit frequency uses a multiplier and two shifts per symbol
-// (T. Granlund, P. Montgomery, "Division by invariant integers using
-// multiplication", PLDI 1994, fig. 4.1).
+// Division x / f by the 12-bit frequency is one high product and a shift, rounded up or down
+// per symbol (A. D. Robison, "N-bit unsigned division via N-bit multiply-add", ARITH 2005).
+//
+// What bounds them (256 CUs; us before and after the present form, 134 M symbols of 3 bits in
+// 2048 blocks / 33.5 M of 8 bits in 512 blocks).  Encoding, 112 -> 79 / 52 -> 32: the vector
+// units' issue at 8 waves a SIMD (instructions per symbol count: table fields where an
+// instruction takes them without an extract, two 32-bit products less), the latency of a step
+// at 2.  Decoding, 92 -> 76 / 45 -> 37.5: a step is two dependent LDS reads and a dozen
+// dependent instructions; at 8 waves a SIMD its LDS conflicts (random table slots) and issue
+// overlap only in part.  The workgroup's LDS stays under 20 KB so that a CU holds 8 and 2048
+// blocks run as one round; the words, header, counts, states and first refill are requested
+// ahead of their use.  Doubles for the quotient (one conversion and one fused multiply-add
+// instead of a 32-bit high product) measured the same as the integers, 84 against 81 us.
 #include "kvmi_device.hpp"
 #include "../../include/kvserve_amd.h"
 
@@ -194,12 +204,41 @@ __device__ __forceinline__ int job_of(const Batch& bt, uint32_t g) {
 // ------------------------------------------------------------------ encode
 constexpr uint32_t kEncGroup = 8;  // steps whose table reads are issued together
 
+// Encoder entry of a symbol of frequency f and cumulative frequency c.  The state's step
+// (x / f) * 4096 + x % f + c is x + (x / f) * (4096 - f) + c, and the quotient is
+// umulhi(m, x + inc) >> s: with s = floor(log2 f) and m the ceiling (inc = 0) or the floor
+// (inc = 1) of 2^(32+s) / f.  A renormalised state is below f * 2^20, for which one of the two
+// is exact: the ceiling's excess e = m f - 2^(32+s) may be up to 2^(12+s) / f, and so may the
+// floor's shortfall f - e; the smaller of them is at most f / 2 < 2^(12+s) / f.  f = 1 takes
+// the floor with m = 2^32 - 1, other powers of two 2^31 and one shift less.
+//   x = m, y = inc, z = c | (f << 4) << 16 (a state emits a word from x >> 16 >= f << 4 on; a
+//   lone symbol's state never does), w = 4096 - f | s << 24.
+// The fields sit where one instruction reads them without an extract (byte and word selects,
+// 24-bit multiply-add).
+__device__ __forceinline__ uint4 enc_entry(uint32_t f, uint32_t cum) {
+  if (f == 0) return make_uint4(0, 0, 0, 0);
+  uint32_t s = 31u - (uint32_t)__clz(f), m, inc = 0;
+  if (f == 1) {
+    m = 0xffffffffu;
+    inc = 1;
+  } else if ((f & (f - 1u)) == 0) {
+    m = 0x80000000u;
+    --s;
+  } else {
+    const uint64_t p = (uint64_t)1 << (32u + s), up = p / f + 1u;
+    const uint32_t e = (uint32_t)(up * f - p);
+    inc = (e * f > (1u << (12u + s))) ? 1u : 0u;
+    m = (uint32_t)up - inc;
+  }
+  return make_uint4(m, inc, cum | (f == kM ? 0xffffu : f << 4) << 16, (kM - f) | (s << 24));
+}
+
 // Steps 255..0 of one sub-block whose runs are block runs run0 .. run0 + 7 (FULL:
 // every lane has a symbol at every step).  Leaves pos < 0 when the words outgrow the
 // capacity (the block is then stored raw).
 template <int W, bool FULL>
 __device__ __forceinline__ void encode_runs(const uint8_t* blk, uint64_t avail, uint32_t run0, uint32_t lane,
-                                            uint32_t nb, const uint2* tab, uint16_t* words, int32_t& pos,
+                                            uint32_t nb, const uint4* tab, uint16_t* words, int32_t& pos,
                                             uint32_t& x) {
   uint32_t d[W], dn[W];
   load_run<W>(blk, avail, run0 + kSubRuns - 1, lane, d);
@@ -208,30 +247,30 @@ __device__ __forceinline__ void encode_runs(const uint8_t* blk, uint64_t avail, 
     const uint32_t base = (run0 + (uint32_t)r) * (kLanes * kRun) + lane * kRun;
 #pragma unroll
     for (int g = (int)kRun / kEncGroup - 1; g >= 0; --g) {
-    // a group's table entries depend on its symbols only: their reads are in flight
-    // before its first step, off the state's dependency chain
-    uint2 ent[kEncGroup];
+      // a group's table entries depend on its symbols only: their reads are in flight
+      // before its first step, off the state's dependency chain
+      uint4 ent[kEncGroup];
 #pragma unroll
-    for (int jj = 0; jj < (int)kEncGroup; ++jj) ent[jj] = tab[sym_at<W>(d, g * (int)kEncGroup + jj)];
+      for (int jj = 0; jj < (int)kEncGroup; ++jj) ent[jj] = tab[sym_at<W>(d, g * (int)kEncGroup + jj)];
 #pragma unroll
-    for (int jj = (int)kEncGroup - 1; jj >= 0; --jj) {
-      const int j = g * (int)kEncGroup + jj;
-      const bool valid = FULL || base + (uint32_t)j < nb;
-      const uint2 e = ent[jj];
-      const uint32_t fs = e.x & 0x1fffu;
-      const bool emit = valid && (x >> 20) >= fs;
-      const uint64_t mask = __ballot(emit);
-      pos -= (int32_t)__popcll(mask);
-      if (emit) {
-        gst16(words + pos + (int32_t)rank_in(mask), x & 0xffffu);
-        x >>= 16;
+      for (int jj = (int)kEncGroup - 1; jj >= 0; --jj) {
+        const int j = g * (int)kEncGroup + jj;
+        const bool valid = FULL || base + (uint32_t)j < nb;
+        const uint4 e = ent[jj];
+        const bool emit = valid && (x >> 16) >= (e.z >> 16);
+        const uint64_t mask = __ballot(emit);
+        pos -= (int32_t)__popcll(mask);
+        if (emit) {
+          gst16(words + pos + rank_in(mask), x & 0xffffu);
+          x >>= 16;
+        }
+        if (valid) {
+          const uint32_t q = __umulhi(e.x, x + e.y) >> (e.w >> 24);
+          uint32_t t = x + (e.z & 0xffffu);
+          asm("" : "+v"(t));  // one word-select add, then one 24-bit multiply-add
+          x = __umul24(q, e.w) + t;
+        }
       }
-      if (valid) {
-        const uint32_t t1 = __umulhi(e.y, x);
-        const uint32_t q = (t1 + ((x - t1) >> ((e.x >> 25) & 1u))) >> (e.x >> 26);
-        x = (q << kPB) + (x - q * fs) + ((e.x >> 13) & 0xfffu);
-      }
-    }
     }
     if (pos < 0) return;
 #pragma unroll
@@ -242,14 +281,15 @@ __device__ __forceinline__ void encode_runs(const uint8_t* blk, uint64_t avail, 
 template <int W>
 __global__ __launch_bounds__(kBlockThreads) void rans_encode_kernel(const EncBatch bt) {
   using G = RansGeo<W>;
-  constexpr bool kPrivate = W <= 5;  // lane-private histogram columns (no LDS contention)
-  constexpr uint32_t kHist = kPrivate ? G::A * kLanes : G::A;  // per wave
-  __shared__ __align__(16) uint32_t hist[kSubs * kHist];
-  __shared__ uint2 tab[G::A];
+  // Histogram columns: one a lane, and half as many at 8 bits (32 KB), so that the lanes of an
+  // atomic hit a bank each; the four waves share them, as their atomics follow each other anyhow
+  constexpr uint32_t kCols = W <= 7 ? kLanes : kLanes / 2;
+  __shared__ __align__(16) uint32_t hist[G::A * kCols];
+  __shared__ uint4 tab[G::A];
   __shared__ uint32_t red[kSubs];
   __shared__ int32_t cnt[kSubs];
 
-  const uint32_t lane = lane_id(), wave = threadIdx.x / kLanes, t = threadIdx.x;
+  const uint32_t lane = lane_id(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kLanes), t = threadIdx.x;
   const int jb = job_of(bt, blockIdx.x);
   const uint64_t n = bt.n[jb];
   const uint64_t b = blockIdx.x - bt.first[jb];
@@ -262,10 +302,10 @@ __global__ __launch_bounds__(kBlockThreads) void rans_encode_kernel(const EncBat
   const uint32_t run0 = wave * kSubRuns;                    // this wave's sub-block
   const bool full = (wave + 1) * kSub <= nb;
 
-  for (uint32_t i = t; i < kSubs * kHist; i += kBlockThreads) hist[i] = 0;
+  for (uint32_t i = t; i < G::A * kCols / 4; i += kBlockThreads) reinterpret_cast<uint4*>(hist)[i] = make_uint4(0, 0, 0, 0);
   __syncthreads();
   {
-    uint32_t* h = hist + wave * kHist;
+    uint32_t* h = hist + lane % kCols;
     uint32_t d[W], dn[W];
     load_run<W>(blk, avail, run0, lane, d);
     for (uint32_t r = 0; r < kSubRuns; ++r) {
@@ -274,7 +314,7 @@ __global__ __launch_bounds__(kBlockThreads) void rans_encode_kernel(const EncBat
 #pragma unroll
       for (int j = 0; j < (int)kRun; ++j) {
         const uint32_t s = sym_at<W>(d, j);
-        if (full || base + (uint32_t)j < nb) atomicAdd(&h[kPrivate ? s * kLanes + lane : s], 1u);
+        if (full || base + (uint32_t)j < nb) atomicAdd(&h[s * kCols], 1u);
       }
 #pragma unroll
       for (int k = 0; k < W; ++k) d[k] = dn[k];
@@ -285,16 +325,10 @@ __global__ __launch_bounds__(kBlockThreads) void rans_encode_kernel(const EncBat
   // thread v < A: count of symbol v over the block
   uint32_t c = 0;
   if (t < G::A) {
-    for (uint32_t j = 0; j < kSubs; ++j) {
-      if (kPrivate) {
-        const uint4* row = reinterpret_cast<const uint4*>(&hist[j * kHist + t * kLanes]);
-        for (int q = 0; q < (int)kLanes / 4; ++q) {
-          const uint4 hv = row[q];
-          c += hv.x + hv.y + hv.z + hv.w;
-        }
-      } else {
-        c += hist[j * kHist + t];
-      }
+    const uint4* row = reinterpret_cast<const uint4*>(&hist[t * kCols]);
+    for (uint32_t q = 0; q < kCols / 4; ++q) {
+      const uint4 hv = row[(q + t) % (kCols / 4)];  // neighbours' rows lie on the same banks
+      c += hv.x + hv.y + hv.z + hv.w;
     }
   }
   const uint32_t K = block_sum(c ? 1u : 0u, red);
@@ -305,12 +339,7 @@ __global__ __launch_bounds__(kBlockThreads) void rans_encode_kernel(const EncBat
   if (t == top) f += kM - fsum;
   if (t < G::A) gst16(reinterpret_cast<uint16_t*>(slot + 4) + t, f);
   const uint32_t cum = block_exclusive_scan(f, red);  // f = 0 for threads >= A
-  if (t < G::A) {
-    const uint32_t l = f <= 1u ? 0u : 32u - __clz(f - 1u);
-    const uint32_t mul = f ? (uint32_t)((((uint64_t)((1u << l) - f)) << 32) / f + 1u) : 0u;
-    const uint32_t sh1 = l ? 1u : 0u, sh2 = l ? l - 1u : 0u;
-    tab[t] = make_uint2(f | (cum << 13) | (sh1 << 25) | (sh2 << 26), mul);
-  }
+  if (t < G::A) tab[t] = enc_entry(f, cum);
   __syncthreads();
 
   // encode, steps 255..0; words fill the sub-block's word region from its end.  The
@@ -466,71 +495,100 @@ __global__ __launch_bounds__(kCopyThreads) void rans_compact_kernel(const EncBat
 }
 
 // ------------------------------------------------------------------ decode
-// A sub-block's words are staged through its wave's LDS ring of kRing 16-bit units,
-// refilled 256 units at a time (two coalesced dword loads per lane) so that a step
-// reads its words from LDS instead of waiting on a dependent global load.
-constexpr uint32_t kRing = 512;
-constexpr uint32_t kRefill = 256;
+// A sub-block's words are staged through its wave's LDS ring of kRing 16-bit units, refilled
+// kRefill units at a time (one coalesced dword a lane, loaded a refill ahead into a register),
+// so that a step reads its words from LDS instead of waiting on a dependent global load.
+constexpr uint32_t kRing = 256;
+constexpr uint32_t kRefill = 2 * kLanes;
+constexpr uint32_t kMirror = kLanes;  // the ring's first units again behind its end: a step reads without wrapping
 
-// Stage units [filled, ...) of the word region into the ring until `want` units
-// (or all) are staged; each pass stages 256 units, two dwords per lane.
-__device__ __forceinline__ void ring_fill(uint16_t* ring, const uint32_t* region, uint32_t units, uint32_t& filled,
-                                          uint32_t want, uint32_t lane) {
-  if (filled >= want || filled >= units) return;
-  do {
-    const uint32_t u = filled + 4u * lane;
-    uint32_t w0 = 0, w1 = 0;
-    if (u < units) w0 = gld(region + u / 2);
-    if (u + 2 < units) w1 = gld(region + u / 2 + 1);
-    uint32_t* rp = reinterpret_cast<uint32_t*>(ring + (u & (kRing - 1)));
-    rp[0] = w0;
-    rp[1] = w1;
-    filled += kRefill;
-  } while (filled < want && filled < units);
+struct RingFeed {
+  const uint32_t* region;
+  uint32_t units;   // of the word region
+  uint32_t filled;  // staged so far
+  uint32_t ahead;   // this lane's dword of the units behind those
+};
+
+__device__ __forceinline__ void ring_ahead(RingFeed& f, uint32_t lane) {
+  const uint32_t u = f.filled + 2u * lane;
+  f.ahead = u < f.units ? gld(f.region + u / 2) : 0u;
+}
+
+// Stages the next kRefill units of the word region unless `want` units (or all) are staged.
+__device__ __forceinline__ void ring_fill(uint16_t* ring, RingFeed& f, uint32_t want, uint32_t lane) {
+  if (f.filled >= want || f.filled >= f.units) return;
+  const uint32_t at = f.filled & (kRing - 1);
+  reinterpret_cast<uint32_t*>(ring + at)[lane] = f.ahead;
+  if (at == 0 && 2u * lane < kMirror) reinterpret_cast<uint32_t*>(ring + kRing)[lane] = f.ahead;
+  f.filled += kRefill;
+  ring_ahead(f, lane);
   wave_lds_fence();
 }
 
 // Steps 0..255 of one sub-block (block runs run0 .. run0 + 7); returns the final
-// state.  Before each group of kGroup steps (at most 64 * kGroup words) the ring
-// holds at least that many unread units.  A refill pass starts only while fewer
-// than 64 * kGroup units are staged past q, and kRing >= 64 * kGroup + kRefill, so
-// it overwrites only units below q.
-constexpr uint32_t kGroup = 4;
+// state.  Before each group of kGroup steps (at most 64 * kGroup words) the ring holds at
+// least that many unread units: a group reads no more than one refill brings, so one is
+// enough.  It starts only while fewer than 64 * kGroup units are staged past q, and kRing >=
+// 64 * kGroup + kRefill, so it overwrites only units below q.
+constexpr uint32_t kGroup = 2;
 static_assert(kRing >= kGroup * kLanes + kRefill, "ring too small for the refill policy");
+static_assert(kRefill >= kGroup * kLanes, "one refill serves a group");
 
-// Decode table: slot -> symbol (bits 0..7), frequency - 1 (8..19) and the slot's
-// offset in its symbol's range (20..31); a step is one LDS read off the state.
+// Decode table: slot -> symbol, frequency and the slot's offset in its symbol's range (bits
+// 20..31); a step is one LDS read off the state.  Up to 7 bits the symbol has bits 0..6 and the
+// frequency 7..19; at 8 bits the symbol needs one more and the frequency is kept less one.
+template <int W>
+__device__ __forceinline__ uint32_t dec_entry(uint32_t sym, uint32_t f, uint32_t off) {
+  return W <= 7 ? sym | f << 7 | off << 20 : sym | (f - 1u) << 8 | off << 20;
+}
+
 template <int W, bool FULL>
-__device__ __forceinline__ uint32_t decode_runs(const uint32_t* region, uint32_t units, uint32_t& q,
-                                                const uint32_t* slot_tab, uint16_t* ring, uint8_t* dst, uint64_t room,
-                                                uint32_t nb, uint32_t run0, uint32_t lane, uint32_t x) {
-  uint32_t filled = 0;
+__device__ __forceinline__ uint32_t decode_runs(RingFeed& feed, uint32_t& q, const uint32_t* slot_tab, uint16_t* ring,
+                                                uint8_t* dst, uint64_t room, uint32_t nb, uint32_t run0, uint32_t lane,
+                                                uint32_t x) {
+  // 32 symbols are packed as they come by shifting each in from the top (one instruction):
+  // kFit whole symbols to a word, then the words are joined
+  constexpr int kFit = 32 / W, kParts = ((int)kRun + kFit - 1) / kFit;
   for (uint32_t r = run0; r < run0 + kSubRuns; ++r) {
-    uint32_t acc[W];
+    uint32_t part[kParts];
 #pragma unroll
-    for (int k = 0; k < W; ++k) acc[k] = 0;
+    for (int k = 0; k < kParts; ++k) part[k] = 0;
     const uint32_t base = r * (kLanes * kRun) + lane * kRun;
 #pragma unroll
     for (int g = 0; g < (int)(kRun / kGroup); ++g) {
-      ring_fill(ring, region, units, filled, q + kGroup * kLanes, lane);
+      ring_fill(ring, feed, q + kGroup * kLanes, lane);
 #pragma unroll
       for (int jj = 0; jj < (int)kGroup; ++jj) {
         const int j = g * (int)kGroup + jj;
         const bool valid = FULL || base + (uint32_t)j < nb;
         const uint32_t ent = slot_tab[x & (kM - 1u)];
-        const uint32_t s = ent & 0xffu;
-        uint32_t y = (((ent >> 8) & 0xfffu) + 1u) * (x >> kPB) + (ent >> 20);
+        const uint32_t t = x >> kPB;
+        uint32_t y = W <= 7 ? __umul24((ent >> 7) & 0x1fffu, t) + (ent >> 20)
+                            : __umul24((ent >> 8) & 0xfffu, t) + (ent >> 20) + t;
         const bool need = valid && y < kStateL;
         const uint64_t mask = __ballot(need);
-        if (need) y = (y << 16) | (uint32_t)ring[(q + rank_in(mask)) & (kRing - 1)];
+        const uint16_t* next = ring + (q & (kRing - 1));
+        // every lane reads (a rank is always inside the ring): cheaper than a branch round the
+        // lanes that need no word, which the compiler would make again of a select alone
+        uint32_t word = next[rank_in(mask)];
+        asm volatile("" : "+v"(word));
+        y = need ? (y << 16) | word : y;
         q += (uint32_t)__popcll(mask);
-        if (valid) {
-          x = y;
-          const int bit = j * W, kk = bit >> 5, sh = bit & 31;
-          acc[kk] |= s << sh;
-          if (sh + W > 32) acc[kk + 1] |= s >> (32 - sh);
-        }
+        x = valid ? y : x;
+        // a lane past the end shifts in zeros, as the packed body is padded
+        part[j / kFit] = __builtin_amdgcn_alignbit(valid ? ent : 0u, part[j / kFit], W);
       }
+    }
+    uint32_t acc[W];
+#pragma unroll
+    for (int k = 0; k < W; ++k) acc[k] = 0;
+#pragma unroll
+    for (int k = 0; k < kParts; ++k) {
+      const int cnt = (k + 1) * kFit <= (int)kRun ? kFit : (int)kRun - k * kFit;  // symbols in this part
+      const uint32_t v = part[k] >> (32 - cnt * W);
+      const int bit = k * kFit * W, kk = bit >> 5, sh = bit & 31;
+      acc[kk] |= v << sh;
+      if (sh + cnt * W > 32) acc[kk + 1] |= v >> (32 - sh);
     }
     const uint64_t off = ((uint64_t)r * kLanes + lane) * (4u * W);
 #pragma unroll
@@ -550,35 +608,40 @@ __device__ __forceinline__ uint32_t decode_runs(const uint32_t* region, uint32_t
 template <int W>
 __global__ __launch_bounds__(kBlockThreads) void rans_decode_kernel(const DecBatch bt, int32_t* __restrict__ err) {
   using G = RansGeo<W>;
-  __shared__ uint32_t slot_tab[kM];
+  __shared__ __align__(16) uint32_t slot_tab[kM];
   __shared__ uint32_t sym_fc[G::A];
   __shared__ uint32_t red[kSubs];
-  __shared__ __align__(16) uint16_t rings[kSubs][kRing];
+  __shared__ __align__(16) uint16_t rings[kSubs][kRing + kMirror];
 
-  const uint32_t lane = lane_id(), wave = threadIdx.x / kLanes, t = threadIdx.x;
+  const uint32_t lane = lane_id(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kLanes), t = threadIdx.x;
   const int jb = job_of(bt, blockIdx.x);
   const uint64_t n = bt.n[jb];
   const uint64_t b = blockIdx.x - bt.first[jb];
   const uint8_t* in = bt.in[jb];
   const uint64_t in_bytes = bt.in_bytes[jb];
   const uint32_t nblk = (uint32_t)((n + kBlock - 1) / kBlock);
-  const uint32_t* h = reinterpret_cast<const uint32_t*>(in);
   const uint64_t head = 32u + 8ull * nblk;
   // Every check below is uniform over the workgroup (it reads the same bytes).  The
   // buffer must hold the header and offset table before any of it is read, and the
   // stated payload is compared with what is left of the buffer (never head + payload,
   // which a payload near 2^64 would wrap).
-  if (in_bytes < head || gld(h) != kRansMagic ||
-      gld(h + 1) != (2u | ((uint32_t)W << 8) | (kPB << 16) | (8u << 24)) || gld(h + 2) != kBlock ||
-      gld(h + 3) != nblk || gld(reinterpret_cast<const uint64_t*>(in + 16)) != n ||
-      gld(reinterpret_cast<const uint64_t*>(in + 24)) > in_bytes - head) {
+  if (in_bytes < head) {
     if (t == 0) atomicOr(err, KVMI_ERR_BAD_HEADER);
     return;
   }
-  const uint64_t payload = gld(reinterpret_cast<const uint64_t*>(in + 24));
+  // the header and the offsets in one trip to memory
+  const uint32_t* h = reinterpret_cast<const uint32_t*>(in);
   const uint64_t* offs = reinterpret_cast<const uint64_t*>(in + 32);
+  const uint32_t h0 = gld(h), h1 = gld(h + 1), h2 = gld(h + 2), h3 = gld(h + 3);
+  const uint64_t hn = gld(reinterpret_cast<const uint64_t*>(in + 16));
+  const uint64_t payload = gld(reinterpret_cast<const uint64_t*>(in + 24));
   const uint64_t o = gld(offs + b);
   const uint64_t e = b + 1 == nblk ? payload : gld(offs + b + 1);
+  if ((h0 ^ kRansMagic) | (h1 ^ (2u | ((uint32_t)W << 8) | (kPB << 16) | (8u << 24))) | (h2 ^ kBlock) | (h3 ^ nblk) |
+      (uint32_t)(hn != n) | (uint32_t)(payload > in_bytes - head)) {
+    if (t == 0) atomicOr(err, KVMI_ERR_BAD_HEADER);
+    return;
+  }
   if (o > e || e > payload || e - o < 4 || (o & 3u)) {
     if (t == 0) atomicOr(err, KVMI_ERR_BAD_HEADER);
     return;
@@ -609,19 +672,34 @@ __global__ __launch_bounds__(kBlockThreads) void rans_decode_kernel(const DecBat
     }
     return;
   }
+  if (e - o < G::kHead) {
+    if (t == 0) atomicOr(err, KVMI_ERR_CORRUPT);
+    return;
+  }
+  // counts, frequencies and states in one trip as well; the first words follow during the
+  // table's build
   uint32_t count[kSubs];
-  uint64_t size = G::kHead;
+#pragma unroll
+  for (uint32_t j = 0; j < kSubs; ++j)
+    count[j] = j ? gld(reinterpret_cast<const uint32_t*>(blk + G::kCounts) + (j - 1)) : tag >> 1;
+  const uint32_t fv = t < G::A ? gld(reinterpret_cast<const uint16_t*>(blk + 4) + t) : 0u;
+  uint32_t x = gld(reinterpret_cast<const uint32_t*>(blk + G::kStates) + wave * kLanes + lane);
+  uint64_t size = G::kHead, region_off = G::kHead;
 #pragma unroll
   for (uint32_t j = 0; j < kSubs; ++j) {
-    count[j] = j ? gld(reinterpret_cast<const uint32_t*>(blk + G::kCounts) + (j - 1)) : tag >> 1;
+    if (j == wave) region_off = size;
     size += pad4(2ull * count[j]);
   }
   if (e - o != size) {
     if (t == 0) atomicOr(err, KVMI_ERR_CORRUPT);
     return;
   }
-  const uint16_t* ftab = reinterpret_cast<const uint16_t*>(blk + 4);
-  const uint32_t fv = t < G::A ? gld(ftab + t) : 0u;
+  // sub-block `wave`: its word region (pad4(2 count) bytes, the words at its end; q counts
+  // 16-bit units from the region start)
+  const uint32_t cw = count[0] * (wave == 0) + count[1] * (wave == 1) + count[2] * (wave == 2) + count[3] * (wave == 3);
+  RingFeed feed{reinterpret_cast<const uint32_t*>(blk + region_off), (uint32_t)(pad4(2ull * cw) / 2), 0, 0};
+  uint32_t q = feed.units - cw;
+  ring_ahead(feed, lane);
   if (block_sum(fv, red) != kM) {
     if (t == 0) atomicOr(err, KVMI_ERR_CORRUPT);
     return;
@@ -629,50 +707,42 @@ __global__ __launch_bounds__(kBlockThreads) void rans_decode_kernel(const DecBat
   const uint32_t cum = block_exclusive_scan(fv, red);
   if (t < G::A) sym_fc[t] = fv | (cum << 13);
   __syncthreads();
-  // slot -> (symbol, frequency, offset): thread i fills slots [16 i, 16 i + 16),
-  // walking the cumulative table
+  // slot -> (symbol, frequency, offset): thread i fills the slots 4 i .. 4 i + 3 of each
+  // quarter.  The symbol of slot s is the last v with cum_v <= s (cum is non-decreasing, and an
+  // absent symbol shares its cum with the next one, so it is never the last): the search runs
+  // for the four quarters side by side, then each walks on over its slots.
   {
-    constexpr uint32_t kPer = kM / kBlockThreads;
-    const uint32_t s0 = t * kPer;
-    // the symbol of slot s is the last v with cum_v <= s (cum is non-decreasing, and
-    // an absent symbol shares its cum with the next one, so it is never the last)
-    uint32_t lo = 0, hi = G::A - 1;
-    while (lo < hi) {
-      const uint32_t mid = (lo + hi + 1) / 2;
-      if ((sym_fc[mid] >> 13) <= s0) lo = mid;
-      else hi = mid - 1;
+    constexpr uint32_t kQuad = kM / (4u * kBlockThreads);
+    uint32_t v[kQuad];
+#pragma unroll
+    for (uint32_t k = 0; k < kQuad; ++k) v[k] = 0;
+#pragma unroll
+    for (uint32_t step = G::A / 2; step > 0; step >>= 1) {
+#pragma unroll
+      for (uint32_t k = 0; k < kQuad; ++k)
+        if ((sym_fc[v[k] + step] >> 13) <= 4u * (t + k * kBlockThreads)) v[k] += step;
     }
-    uint32_t v = lo;
-    uint32_t end = (sym_fc[v] >> 13) + (sym_fc[v] & 0x1fffu);
-    for (uint32_t s = s0; s < s0 + kPer; ++s) {
-      while (s >= end) {
-        ++v;
-        end = (sym_fc[v] >> 13) + (sym_fc[v] & 0x1fffu);
+#pragma unroll
+    for (uint32_t k = 0; k < kQuad; ++k) {
+      const uint32_t s0 = 4u * (t + k * kBlockThreads);
+      uint32_t fc = sym_fc[v[k]], ent[4];
+#pragma unroll
+      for (uint32_t i = 0; i < 4; ++i) {
+        while (s0 + i >= (fc >> 13) + (fc & 0x1fffu)) fc = sym_fc[++v[k]];
+        ent[i] = dec_entry<W>(v[k], fc & 0x1fffu, s0 + i - (fc >> 13));
       }
-      const uint32_t fv = sym_fc[v] & 0x1fffu, cum = sym_fc[v] >> 13;
-      slot_tab[s] = v | ((fv - 1u) << 8) | ((s - cum) << 20);
+      reinterpret_cast<uint4*>(slot_tab)[t + k * kBlockThreads] = make_uint4(ent[0], ent[1], ent[2], ent[3]);
     }
   }
   __syncthreads();
 
-  // sub-block `wave`: its states, and its word region (pad4(2 count) bytes, the words
-  // at its end; q counts 16-bit units from the region start)
-  uint32_t x = gld(reinterpret_cast<const uint32_t*>(blk + G::kStates) + wave * kLanes + lane);
-  uint64_t region_off = G::kHead;
-#pragma unroll
-  for (uint32_t j = 0; j < kSubs; ++j)
-    if (j < wave) region_off += pad4(2ull * count[j]);
-  const uint32_t cw = count[0] * (wave == 0) + count[1] * (wave == 1) + count[2] * (wave == 2) + count[3] * (wave == 3);
-  const uint32_t* region = reinterpret_cast<const uint32_t*>(blk + region_off);
-  const uint32_t units = (uint32_t)(pad4(2ull * cw) / 2);
-  uint32_t q = units - cw;
   const uint32_t run0 = wave * kSubRuns;
   uint16_t* ring = rings[wave];
-  if ((wave + 1) * kSub <= nb) x = decode_runs<W, true>(region, units, q, slot_tab, ring, dst, room, nb, run0, lane, x);
-  else x = decode_runs<W, false>(region, units, q, slot_tab, ring, dst, room, nb, run0, lane, x);
+  if ((wave + 1) * kSub <= nb) x = decode_runs<W, true>(feed, q, slot_tab, ring, dst, room, nb, run0, lane, x);
+  else x = decode_runs<W, false>(feed, q, slot_tab, ring, dst, room, nb, run0, lane, x);
   // a stream that is not this block's own encoding ends off its start state or
   // off the end of its words (ring reads are masked, so none leaves the ring)
-  const bool ok = q == units && x == kStateL;
+  const bool ok = q == feed.units && x == kStateL;
   if (__ballot(!ok) && lane == 0) atomicOr(err, KVMI_ERR_CORRUPT);
 }
 
