@@ -355,168 +355,111 @@ __global__ __launch_bounds__(kRtThreads) void rt_hadamard_kernel(const uint16_t*
 }
 
 // ================================================================== row kernels
-// One wave per canonical row (all heads of one token of one layer).  A head row of D
-// channels spans LH = D / E lanes holding E contiguous channels each; a wave pass
-// covers HPW = 64 / LH heads and P passes cover the row.  Loads and stores are E-wide
-// vectors, the FWHT runs in registers (in-lane stages, then lane xor stages), and the
-// transformed rows never leave the chip: the token axis reduces inside the wave, the
-// channel / tensor axes take a statistics pass (per-workgroup partials) and a small
-// reduction before the quantizing pass.
+// A wave takes rows_per_wave consecutive canonical rows (all heads of one token of one
+// layer).  A head row of D channels spans LH = D / 8 lanes holding 8 contiguous channels
+// each; a wave pass covers HPW = 64 / LH heads and P passes cover the row.  The rows' loads
+// are issued together and wait packed, as they came; then each row is transformed in
+// registers (in-lane stages, then lane xor stages), and the transformed rows never leave the
+// chip: the token axis reduces inside the wave, the channel / tensor axes take a statistics
+// pass (per-workgroup partials) and a small reduction before the quantizing pass.
+//
+// What bounds them: the transform's roundings (a conversion issues at half rate, eight to a
+// value) and, each alone about as long, the trips to memory in front of a row (layer, block id,
+// row) with the bytes themselves; without the transform the kernels below take 13, 16 and 12 us.
+// So a wave's index is a scalar and the layer's description lies in scalar registers, values
+// wait as bf16 pairs so that 7 or 8 waves fit a SIMD, a rounding is one instruction and every
+// lane step up to 8 a DPP move.  28 layers x 1024 rows of 4 x 128 (29 MB of cache, 15 MB of
+// symbols), before and after: statistics 25 -> 21.5 us with 4 times the workgroups, their
+// reduction 11 -> 4.7, encode 27.6 -> 26.4, decode 23.4 -> 23.1.
 template <int D>
 struct RowGeo {
-  static constexpr int E = D <= 8 ? D : (D / 64 > 8 ? D / 64 : 8);
-  static constexpr int LH = D / E;
+  static constexpr int LH = D / 8;
   static constexpr int HPW = 64 / LH;
 };
 
-constexpr int kStatRows = 64;     // rows per workgroup of the statistics pass
+constexpr int E = 8;              // channels a lane holds of a head row
+constexpr int kStatRows = 16;     // rows per workgroup of the statistics pass
 constexpr int kMaxRowCols = 2048; // H * D held by one wave (<= 32 values per lane)
 
-template <int E>
-__device__ __forceinline__ void ld_seg(const uint16_t* p, float (&v)[E], bool vec) {
+// 8 bf16 values as they lie in memory, two to a dword
+__device__ __forceinline__ uint4 ld_seg(const uint16_t* p, bool vec) {
+  if (vec) return gld(reinterpret_cast<const uint4*>(p));
+  uint32_t w[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) w[i] = (uint32_t)gld(p + 2 * i) | (uint32_t)gld(p + 2 * i + 1) << 16;
+  return make_uint4(w[0], w[1], w[2], w[3]);
+}
+
+__device__ __forceinline__ void st_seg(uint16_t* p, const uint4& t, bool vec) {
   if (vec) {
-    if constexpr (E >= 8) {
-#pragma unroll
-      for (int i = 0; i < E / 8; ++i) {
-        const uint4 t = gld(reinterpret_cast<const uint4*>(p) + i);
-        const uint32_t w[4] = {t.x, t.y, t.z, t.w};
-#pragma unroll
-        for (int j = 0; j < 4; ++j) v[8 * i + 2 * j] = bf_lo(w[j]), v[8 * i + 2 * j + 1] = bf_hi(w[j]);
-      }
-    } else if constexpr (E == 4) {
-      const uint2 t = gld(reinterpret_cast<const uint2*>(p));
-      v[0] = bf_lo(t.x), v[1] = bf_hi(t.x), v[2] = bf_lo(t.y), v[3] = bf_hi(t.y);
-    } else if constexpr (E == 2) {
-      const uint32_t t = gld(reinterpret_cast<const uint32_t*>(p));
-      v[0] = bf_lo(t), v[1] = bf_hi(t);
-    } else {
-      v[0] = ld_bf16(p);
-    }
-  } else {
-#pragma unroll
-    for (int k = 0; k < E; ++k) v[k] = ld_bf16(p + k);
+    gst(reinterpret_cast<uint4*>(p), t);
+    return;
   }
+  const uint32_t w[4] = {t.x, t.y, t.z, t.w};
+#pragma unroll
+  for (int i = 0; i < 4; ++i) gst(p + 2 * i, (uint16_t)w[i]), gst(p + 2 * i + 1, (uint16_t)(w[i] >> 16));
 }
 
-template <int E>
-__device__ __forceinline__ void st_seg(uint16_t* p, const float (&v)[E], bool vec) {
-  if (vec) {
-    if constexpr (E >= 8) {
+__device__ __forceinline__ void unpack_seg(const uint4& t, float (&v)[E]) {
+  const uint32_t w[4] = {t.x, t.y, t.z, t.w};
 #pragma unroll
-      for (int i = 0; i < E / 8; ++i)
-        gst(reinterpret_cast<uint4*>(p) + i,
-            make_uint4(pack_bf16x2(v[8 * i], v[8 * i + 1]), pack_bf16x2(v[8 * i + 2], v[8 * i + 3]),
-                       pack_bf16x2(v[8 * i + 4], v[8 * i + 5]), pack_bf16x2(v[8 * i + 6], v[8 * i + 7])));
-    } else if constexpr (E == 4) {
-      gst(reinterpret_cast<uint2*>(p), make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])));
-    } else if constexpr (E == 2) {
-      gst(reinterpret_cast<uint32_t*>(p), pack_bf16x2(v[0], v[1]));
-    } else {
-      st_bf16(p, v[0]);
-    }
-  } else {
-#pragma unroll
-    for (int k = 0; k < E; ++k) st_bf16(p + k, v[k]);
-  }
+  for (int i = 0; i < 4; ++i) v[2 * i] = bf_lo(w[i]), v[2 * i + 1] = bf_hi(w[i]);
 }
 
-// E u8 symbols, packed 4 per dword
-template <int E>
-__device__ __forceinline__ void ld_sym(const uint8_t* p, uint32_t (&w)[(E + 3) / 4]) {
-  if constexpr (E >= 8) {
-#pragma unroll
-    for (int i = 0; i < E / 8; ++i) {
-      const uint2 t = gld(reinterpret_cast<const uint2*>(p) + i);
-      w[2 * i] = t.x, w[2 * i + 1] = t.y;
-    }
-  } else if constexpr (E == 4) {
-    w[0] = gld(reinterpret_cast<const uint32_t*>(p));
-  } else {
-    w[0] = 0;
-#pragma unroll
-    for (int k = 0; k < E; ++k) w[0] |= (uint32_t)gld(p + k) << (8 * k);
-  }
+// values that are bf16 already
+__device__ __forceinline__ uint4 pack_seg(const float (&v)[E]) {
+  return make_uint4(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]), pack_bf16x2(v[4], v[5]), pack_bf16x2(v[6], v[7]));
 }
 
-template <int E>
-__device__ __forceinline__ void st_sym(uint8_t* p, const uint32_t (&w)[(E + 3) / 4]) {
-  if constexpr (E >= 8) {
-#pragma unroll
-    for (int i = 0; i < E / 8; ++i) gst(reinterpret_cast<uint2*>(p) + i, make_uint2(w[2 * i], w[2 * i + 1]));
-  } else if constexpr (E == 4) {
-    gst(reinterpret_cast<uint32_t*>(p), w[0]);
-  } else {
-#pragma unroll
-    for (int k = 0; k < E; ++k) gst(p + k, (uint8_t)(w[0] >> (8 * k)));
-  }
+__device__ __forceinline__ uint4 xor_seg(const uint4& a, const uint4& b) {
+  return make_uint4(a.x ^ b.x, a.y ^ b.y, a.z ^ b.z, a.w ^ b.w);
 }
 
-// Signs of a head row: bf16 +-1, applied as the exact sign flip x * s.
-template <int E>
-__device__ __forceinline__ void mul_signs(float (&v)[E], const uint16_t* s) {
-  float sg[E];
-  ld_seg<E>(s, sg, true);
-#pragma unroll
-  for (int k = 0; k < E; ++k) v[k] = __uint_as_float(__float_as_uint(v[k]) ^ (__float_as_uint(sg[k]) & 0x80000000u));
+// x rounded to bf16 in one instruction: the conversion of (0, x) leaves x's value in place
+__device__ __forceinline__ float rn1(float x) { return __uint_as_float(pack_bf16x2(0.0f, x)); }
+
+// The lane steps of the transform as moves a DPP has: 1 and 2 within a quad, 7 (a half row
+// mirrored), 8, then 16 by a swizzle.  Channel group `sub` of a head row lies in the lane
+// whose index is the exclusive or of the steps of sub's bits, so bit 2 of a lane's place flips
+// the two below it.
+template <int J>
+__device__ __forceinline__ float row_step(float x) {
+  if constexpr (J == 4) return dpp_f<0x141>(x);
+  else return lane_xor<J>(x);
 }
 
-// x and y rounded to bf16 with one conversion instruction
-__device__ __forceinline__ void rn2(float& x, float& y) {
-  const uint32_t p = pack_bf16x2(x, y);
-  x = bf_lo(p);
-  y = bf_hi(p);
-}
-
-// Butterfly stages across lanes J, 2J, .. < LH: the lane with bit J clear holds the
+// Butterfly stages across lane groups J, 2J, .. < LH: the lane with bit J clear holds the
 // lower element a and gets a + b, the other gets a - b = partner - own; fma(v, +-1, o)
 // is that sum with one fp32 rounding, then bf16.
-template <int J, int LH, int P, int E>
-__device__ __forceinline__ void fwht_cross(float (&v)[P][E], uint32_t lane) {
+template <int J, int LH>
+__device__ __forceinline__ void fwht_cross(float (&v)[E], uint32_t sub) {
   if constexpr (J < LH) {
-    const float sgn = (lane & J) ? -1.0f : 1.0f;
+    const float sgn = (sub & J) ? -1.0f : 1.0f;
 #pragma unroll
-    for (int p = 0; p < P; ++p) {
-#pragma unroll
-      for (int k = 0; k < E; ++k) v[p][k] = __builtin_fmaf(v[p][k], sgn, lane_xor<J>(v[p][k]));
-#pragma unroll
-      for (int k = 0; k < E; k += 2) rn2(v[p][k], v[p][k + 1]);
-    }
-    fwht_cross<J * 2, LH, P, E>(v, lane);
+    for (int k = 0; k < E; ++k) v[k] = rn1(__builtin_fmaf(v[k], sgn, row_step<J>(v[k])));
+    fwht_cross<J * 2, LH>(v, sub);
   }
 }
 
-template <int D, int P>
-__device__ __forceinline__ void fwht_rows(float (&v)[P][RowGeo<D>::E], uint32_t lane, float scale) {
-  constexpr int E = RowGeo<D>::E, LH = RowGeo<D>::LH;
-  static_assert(E % 2 == 0, "pairs of elements per lane");
+template <int D>
+__device__ __forceinline__ void fwht_seg(float (&v)[E], uint32_t sub, float scale) {
 #pragma unroll
   for (int m = 1; m < E; m <<= 1) {
 #pragma unroll
-    for (int p = 0; p < P; ++p) {
-#pragma unroll
-      for (int k = 0; k < E; ++k) {
-        if (k & m) continue;
-        const float a = v[p][k], b = v[p][k | m];
-        v[p][k] = a + b;
-        v[p][k | m] = a - b;
-        rn2(v[p][k], v[p][k | m]);
-      }
+    for (int k = 0; k < E; ++k) {
+      if (k & m) continue;
+      const float a = v[k], b = v[k | m];
+      v[k] = rn1(a + b);
+      v[k | m] = rn1(a - b);
     }
   }
-  fwht_cross<1, LH, P, E>(v, lane);
+  fwht_cross<1, RowGeo<D>::LH>(v, sub);
 #pragma unroll
-  for (int p = 0; p < P; ++p) {
-#pragma unroll
-    for (int k = 0; k < E; k += 2) {
-      v[p][k] *= scale;
-      v[p][k + 1] *= scale;
-      rn2(v[p][k], v[p][k + 1]);
-    }
-  }
+  for (int k = 0; k < E; ++k) v[k] = rn1(v[k] * scale);
 }
 
 struct RowLane {
-  uint32_t lane, slot, sub;  // lane, head slot of the pass, lane within the head row
+  uint32_t lane, slot, sub;  // lane, head slot of the pass, channel group within the head row
 };
 
 template <int D>
@@ -525,131 +468,130 @@ __device__ __forceinline__ RowLane row_lane() {
   r.lane = threadIdx.x & 63;
   r.slot = r.lane / RowGeo<D>::LH;
   r.sub = r.lane % RowGeo<D>::LH;
+  if (RowGeo<D>::LH >= 8 && (r.lane & 4)) r.sub ^= 3;
   return r;
 }
 
-// Rows whose loads a wave issues together: 4 rows of one pass, fewer for wider rows
-// (the values of R rows x P passes stay in registers).
-template <int P>
-constexpr int rows_per_wave() { return P >= 4 ? 1 : 4 / P; }
+__device__ __forceinline__ uint32_t wave_index() { return __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); }
 
-// Per-wave constants of one layer: the cache head of each pass (-1: no head in this
-// slot) and the signs of the lane's channels.
+// Rows whose loads a wave issues together: 4 rows of one pass in the statistics, fewer for
+// wider rows; half of that where a row is also written, whose waves then come in more rounds
+// that overlap (encode 27.6 against 26.4 us, decode 24.4 against 23.1).
+template <int P>
+constexpr int stat_rows_per_wave() { return P >= 4 ? 1 : 4 / P; }
+template <int P>
+constexpr int rows_per_wave() { return P >= 2 ? 1 : 2; }
+
+// Per-lane constants of one layer: the cache head of each pass (-1: no head in this
+// slot) and the sign bits of the lane's channels (signs are bf16 +-1: an exact flip).
 template <int D, int P>
 struct LayerLanes {
   int hc[P];
-  float sg[P][RowGeo<D>::E];
+  uint4 flip[P];
 };
 
 template <int D, int P>
 __device__ __forceinline__ void layer_lanes(const kvmi_rt_geometry& g, const kvmi_rt_layer& L, const RowLane& rl,
                                             LayerLanes<D, P>& c) {
-  constexpr int E = RowGeo<D>::E, HPW = RowGeo<D>::HPW;
   const uint16_t* signs = static_cast<const uint16_t*>(L.signs);
 #pragma unroll
   for (int p = 0; p < P; ++p) {
-    const int h = p * HPW + (int)rl.slot;
+    const int h = p * RowGeo<D>::HPW + (int)rl.slot;
     c.hc[p] = h < g.num_heads ? gld(L.head_order + h) : -1;
+    c.flip[p] = make_uint4(0, 0, 0, 0);
     if (signs && h < g.num_heads) {
-      ld_seg<E>(signs + (int64_t)h * D + rl.sub * E, c.sg[p], true);
-    } else {
-#pragma unroll
-      for (int k = 0; k < E; ++k) c.sg[p][k] = 1.0f;
+      const uint4 t = ld_seg(signs + (int64_t)h * D + rl.sub * E, true);
+      constexpr uint32_t kS = 0x80008000u;
+      c.flip[p] = make_uint4(t.x & kS, t.y & kS, t.z & kS, t.w & kS);
     }
   }
 }
 
-// Physical block and token of row row0 + lane (lanes < n), for the rows a wave
-// handles; lane j's pair is broadcast when row j is processed.
-struct RowRef {
-  int64_t pb;
-  uint32_t tok;
-};
-
-__device__ __forceinline__ RowRef row_ref(const kvmi_rt_geometry& g, const int64_t* block_ids, uint32_t row0,
-                                          uint32_t n, uint32_t lane) {
-  RowRef r = {0, 0};
-  if (lane < n) {
-    const uint32_t row = row0 + lane, kt = (uint32_t)g.kernel_tokens;
-    const uint32_t blk = row / kt;
-    r.tok = row - blk * kt;
-    r.pb = gld(block_ids + blk);
-  }
-  return r;
+// Element offset in the cache of row row0 + lane (lanes < n), for the rows a wave handles;
+// lane j's is broadcast for row j.
+__device__ __forceinline__ int64_t row_ref(const kvmi_rt_geometry& g, const kvmi_rt_layer& L, const int64_t* block_ids,
+                                           uint32_t row0, uint32_t n, uint32_t lane) {
+  if (lane >= n) return 0;
+  const uint32_t row = row0 + lane, kt = (uint32_t)g.kernel_tokens;
+  const uint32_t blk = row / kt;
+  return gld(block_ids + blk) * L.block_stride + (int64_t)(row - blk * kt) * L.token_stride;
 }
 
-// gather -> signs -> [FWHT] of rows row0 .. row0 + n - 1 (n <= R) into v, in output-head
-// order; `pbl` holds the rows' physical blocks in lanes 0 .. n - 1.  The cache loads of
-// all R rows are issued before any of them is used.
+__device__ __forceinline__ int64_t row_at(int64_t ref, uint32_t j) {
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)ref, j);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)((uint64_t)ref >> 32), j);
+  return (int64_t)((uint64_t)hi << 32 | lo);
+}
+
+// Rows row0 .. row0 + n - 1 (n <= R) of the cache in output-head order, `ref` holding their
+// offsets in lanes first .. first + n - 1; all loads are issued before any is used.
 template <int D, int P, int R>
-__device__ __forceinline__ void load_rows(const kvmi_rt_geometry& g, const kvmi_rt_layer& L,
-                                          const LayerLanes<D, P>& c, const RowRef& ref, uint32_t n,
-                                          const RowLane& rl, float (&v)[R][P][RowGeo<D>::E], bool vec, float scale) {
-  constexpr int E = RowGeo<D>::E;
-  const uint16_t* base = static_cast<const uint16_t*>(L.cache) + L.channel_offset + rl.sub * E;
+__device__ __forceinline__ void fetch_rows(const kvmi_rt_layer& L, const LayerLanes<D, P>& c, int64_t ref, uint32_t first,
+                                           uint32_t n, const RowLane& rl, uint4 (&raw)[R][P], bool vec) {
+  const uint16_t* cache = static_cast<const uint16_t*>(L.cache) + L.channel_offset;
 #pragma unroll
   for (int j = 0; j < R; ++j) {
-    const int64_t pb = __shfl(ref.pb, j, 64);
-    const uint32_t tok = (uint32_t)__shfl((int)ref.tok, j, 64);
-    const uint16_t* row = base + pb * L.block_stride + (int64_t)tok * L.token_stride;
+    const uint16_t* row = cache + row_at(ref, first + j);
 #pragma unroll
     for (int p = 0; p < P; ++p) {
-      if ((uint32_t)j < n && c.hc[p] >= 0) {
-        ld_seg<E>(row + (int64_t)c.hc[p] * L.head_stride, v[j][p], vec);
-      } else {
-#pragma unroll
-        for (int k = 0; k < E; ++k) v[j][p][k] = 0.0f;
-      }
+      raw[j][p] = make_uint4(0, 0, 0, 0);
+      if ((uint32_t)j < n && c.hc[p] >= 0) raw[j][p] = ld_seg(row + (c.hc[p] * L.head_stride + rl.sub * E), vec);
     }
-  }
-  if (L.signs) {
-#pragma unroll
-    for (int j = 0; j < R; ++j)
-#pragma unroll
-      for (int p = 0; p < P; ++p)
-#pragma unroll
-        for (int k = 0; k < E; ++k)
-          v[j][p][k] = __uint_as_float(__float_as_uint(v[j][p][k]) ^ (__float_as_uint(c.sg[p][k]) & 0x80000000u));
-  }
-  if (g.flags & KVMI_RT_TRANSFORM) {
-#pragma unroll
-    for (int j = 0; j < R; ++j) fwht_rows<D, P>(v[j], rl.lane, scale);
   }
 }
 
-__device__ __forceinline__ float wave_min(float x) {
+// signs -> [FWHT] of one fetched row
+template <int D, int P>
+__device__ __forceinline__ void transform_row(const kvmi_rt_geometry& g, const LayerLanes<D, P>& c, const RowLane& rl,
+                                              const uint4 (&raw)[P], float (&v)[P][E], float scale) {
 #pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) x = fminf(x, __shfl_xor(x, o, 64));
-  return x;
+  for (int p = 0; p < P; ++p) {
+    unpack_seg(xor_seg(raw[p], c.flip[p]), v[p]);
+    if (g.flags & KVMI_RT_TRANSFORM) fwht_seg<D>(v[p], rl.sub, scale);
+  }
+}
+
+// Minimum / maximum over the wave: DPP within a row of 16, then the halves exchanged.
+template <class F>
+__device__ __forceinline__ float wave_reduce(float x, F f) {
+  x = f(x, dpp_f<0xB1>(x));
+  x = f(x, dpp_f<0x4E>(x));
+  x = f(x, dpp_f<0x141>(x));
+  x = f(x, dpp_f<0x140>(x));
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  x = f(__uint_as_float(r[0]), __uint_as_float(r[1]));
+  const auto q = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return f(__uint_as_float(q[0]), __uint_as_float(q[1]));
+}
+__device__ __forceinline__ float wave_min(float x) {
+  return wave_reduce(x, [](float a, float b) { return fminf(a, b); });
 }
 __device__ __forceinline__ float wave_max(float x) {
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) x = fmaxf(x, __shfl_xor(x, o, 64));
-  return x;
+  return wave_reduce(x, [](float a, float b) { return fmaxf(a, b); });
 }
 
 // Statistics pass: per-workgroup min / max of every column of the layer's rows
 // [r0, r0 + kStatRows), written as fp32 partials [layer][workgroup][2][cols].  Each
-// wave takes kStatRows / 4 consecutive rows, rows_per_wave at a time.
+// wave takes kStatRows / 4 consecutive rows, stat_rows_per_wave at a time.
 template <int D, int P>
 __global__ __launch_bounds__(kRtThreads) void rt_stats_kernel(kvmi_rt_geometry g, const kvmi_rt_layer* __restrict__ layers,
                                                               const int64_t* __restrict__ block_ids, uint64_t rows,
                                                               float* __restrict__ partial, uint32_t wgs_per_layer,
                                                               bool vec, float scale) {
-  constexpr int E = RowGeo<D>::E, HPW = RowGeo<D>::HPW, R = rows_per_wave<P>();
+  constexpr int HPW = RowGeo<D>::HPW, R = stat_rows_per_wave<P>();
   constexpr uint32_t kWaveRows = kStatRows / kRtWaves;
   static_assert(kWaveRows <= 64 && kWaveRows % R == 0, "one block id per lane");
   __shared__ float smn[kMaxRowCols], smx[kMaxRowCols];
   const uint32_t layer = blockIdx.x / wgs_per_layer, wg = blockIdx.x % wgs_per_layer;
   const kvmi_rt_layer L = layers[layer];
   const RowLane rl = row_lane<D>();
-  const uint32_t wave = threadIdx.x >> 6;
+  const uint32_t wave = wave_index();
   LayerLanes<D, P> c;
   layer_lanes<D, P>(g, L, rl, c);
   const uint32_t nrows = (uint32_t)rows;
   const uint32_t r0 = wg * kStatRows + wave * kWaveRows;
   const uint32_t nw = r0 < nrows ? min(kWaveRows, nrows - r0) : 0u;
-  const RowRef all = row_ref(g, block_ids, r0, nw, rl.lane);
+  const int64_t ref = row_ref(g, L, block_ids, r0, nw, rl.lane);
   float mn[P][E], mx[P][E];
 #pragma unroll
   for (int p = 0; p < P; ++p)
@@ -657,18 +599,17 @@ __global__ __launch_bounds__(kRtThreads) void rt_stats_kernel(kvmi_rt_geometry g
     for (int k = 0; k < E; ++k) mn[p][k] = INFINITY, mx[p][k] = -INFINITY;
   for (uint32_t i = 0; i < nw; i += R) {
     const uint32_t n = min((uint32_t)R, nw - i);
-    RowRef ref;  // lane j: row r0 + i + j
-    ref.pb = __shfl(all.pb, (int)((rl.lane + i) & 63u), 64);
-    ref.tok = (uint32_t)__shfl((int)all.tok, (int)((rl.lane + i) & 63u), 64);
-    float v[R][P][E];
-    load_rows<D, P, R>(g, L, c, ref, n, rl, v, vec, scale);
+    uint4 raw[R][P];
+    fetch_rows<D, P, R>(L, c, ref, i, n, rl, raw, vec);
 #pragma unroll
     for (int j = 0; j < R; ++j) {
       if ((uint32_t)j >= n) break;
+      float v[P][E];
+      transform_row<D, P>(g, c, rl, raw[j], v, scale);
 #pragma unroll
       for (int p = 0; p < P; ++p)
 #pragma unroll
-        for (int k = 0; k < E; ++k) mn[p][k] = fminf(mn[p][k], v[j][p][k]), mx[p][k] = fmaxf(mx[p][k], v[j][p][k]);
+        for (int k = 0; k < E; ++k) mn[p][k] = fminf(mn[p][k], v[p][k]), mx[p][k] = fmaxf(mx[p][k], v[p][k]);
     }
   }
   const uint32_t cols = (uint32_t)g.num_heads * D;
@@ -695,7 +636,52 @@ __global__ __launch_bounds__(kRtThreads) void rt_stats_kernel(kvmi_rt_geometry g
   }
 }
 
-// Reduce the partials of one layer into the channel / tensor section parameters.
+// Reduce the partials of one layer into the channel section parameters: a workgroup takes 64
+// columns, each wave a quarter of the partials.
+__global__ __launch_bounds__(kRtThreads) void rt_stats_channel_kernel(kvmi_rt_geometry g,
+                                                                      const kvmi_rt_layer* __restrict__ layers,
+                                                                      const float* __restrict__ partial,
+                                                                      uint32_t wgs_per_layer, uint32_t col_wgs,
+                                                                      uint8_t* __restrict__ aux, uint64_t half) {
+  __shared__ float smn[kRtWaves][64], smx[kRtWaves][64];
+  const uint32_t layer = blockIdx.x / col_wgs;
+  const kvmi_rt_layer L = layers[layer];
+  const uint32_t D = (uint32_t)g.head_dim, cols = (uint32_t)g.num_heads * D;
+  const uint32_t lane = threadIdx.x & 63, wave = wave_index();
+  const uint32_t c = (blockIdx.x - layer * col_wgs) * 64 + lane;
+  float mn = INFINITY, mx = -INFINITY;
+  if (c < cols) {
+    const float* base = partial + (uint64_t)layer * wgs_per_layer * 2 * cols + c;
+    uint32_t w = wave;
+    for (; w + 7 * kRtWaves < wgs_per_layer; w += 8 * kRtWaves) {  // eight partials in flight
+      float a[8], b[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        a[u] = gld(base + (uint64_t)(w + u * kRtWaves) * 2 * cols);
+        b[u] = gld(base + (uint64_t)(w + u * kRtWaves) * 2 * cols + cols);
+      }
+#pragma unroll
+      for (int u = 0; u < 8; ++u) mn = fminf(mn, a[u]), mx = fmaxf(mx, b[u]);
+    }
+    for (; w < wgs_per_layer; w += kRtWaves) {
+      mn = fminf(mn, gld(base + (uint64_t)w * 2 * cols));
+      mx = fmaxf(mx, gld(base + (uint64_t)w * 2 * cols + cols));
+    }
+  }
+  smn[wave][lane] = mn;
+  smx[wave][lane] = mx;
+  __syncthreads();
+  if (wave != 0 || c >= cols) return;
+#pragma unroll
+  for (int w = 1; w < kRtWaves; ++w) mn = fminf(mn, smn[w][lane]), mx = fmaxf(mx, smx[w][lane]);
+  const int si = section_of(L, (int)(c / D));
+  if (si >= L.num_sections) return;
+  const kvmi_rt_section s = si ? L.sections[1] : L.sections[0];
+  if (s.axis == 0) put_params(aux, half, s, c - (uint32_t)s.head_start * D, quant_params(mn, mx, s.levels));
+}
+
+// The same with tensor sections among the layers', whose parameters need the whole layer: one
+// workgroup a layer.
 __global__ __launch_bounds__(kRtThreads) void rt_stats_reduce_kernel(kvmi_rt_geometry g,
                                                                      const kvmi_rt_layer* __restrict__ layers,
                                                                      const float* __restrict__ partial,
@@ -759,13 +745,6 @@ __global__ __launch_bounds__(kRtThreads) void rt_stats_reduce_kernel(kvmi_rt_geo
     }
 }
 
-// Quantization parameters of a lane's channels for a channel / tensor section (read
-// from aux, constant over the layer's rows), or unused for a token section.
-template <int D, int P>
-struct LaneParams {
-  float mn[P][RowGeo<D>::E], inv[P][RowGeo<D>::E];
-};
-
 // Encode pass: a wave takes rows_per_wave consecutive rows of one layer.  Quantized:
 // token sections reduce inside the wave, channel / tensor sections read their
 // parameters from aux; the u8 symbols land at the layer's u8_offset.  Not quantized:
@@ -776,9 +755,9 @@ __global__ __launch_bounds__(kRtThreads) void rt_row_encode_kernel(kvmi_rt_geome
                                                                    uint32_t num_layers, uint8_t* __restrict__ packed,
                                                                    uint8_t* __restrict__ aux, uint64_t half, bool vec,
                                                                    float scale) {
-  constexpr int E = RowGeo<D>::E, HPW = RowGeo<D>::HPW, R = rows_per_wave<P>();
+  constexpr int HPW = RowGeo<D>::HPW, R = rows_per_wave<P>();
   const uint32_t nrows = (uint32_t)rows, groups = (nrows + R - 1) / R;
-  const uint32_t task = blockIdx.x * kRtWaves + (threadIdx.x >> 6);
+  const uint32_t task = blockIdx.x * kRtWaves + wave_index();
   if (task >= groups * num_layers) return;  // wave-uniform
   const uint32_t layer = task / groups;
   const uint32_t row0 = (task - layer * groups) * R;
@@ -787,44 +766,42 @@ __global__ __launch_bounds__(kRtThreads) void rt_row_encode_kernel(kvmi_rt_geome
   const RowLane rl = row_lane<D>();
   LayerLanes<D, P> c;
   layer_lanes<D, P>(g, L, rl, c);
-  const RowRef ref = row_ref(g, block_ids, row0, n, rl.lane);
-  float v[R][P][E];
-  load_rows<D, P, R>(g, L, c, ref, n, rl, v, vec, scale);
+  uint4 raw[R][P];
+  fetch_rows<D, P, R>(L, c, row_ref(g, L, block_ids, row0, n, rl.lane), 0, n, rl, raw, vec);
   const uint64_t cols = (uint64_t)g.num_heads * D;
   if (!(g.flags & KVMI_RT_QUANTIZE)) {
 #pragma unroll
     for (int j = 0; j < R; ++j) {
       if ((uint32_t)j >= n) break;
-      uint16_t* out = reinterpret_cast<uint16_t*>(packed) + L.u8_offset + (row0 + j) * cols + rl.sub * E;
+      float v[P][E];
+      transform_row<D, P>(g, c, rl, raw[j], v, scale);
+      uint16_t* out = reinterpret_cast<uint16_t*>(packed) + L.u8_offset + (row0 + j) * cols;
 #pragma unroll
       for (int p = 0; p < P; ++p) {
         const int h = p * HPW + (int)rl.slot;
-        if (h < g.num_heads) st_seg<E>(out + (int64_t)h * D, v[j][p], true);
+        if (h < g.num_heads) st_seg(out + ((uint32_t)h * D + rl.sub * E), pack_seg(v[p]), true);
       }
     }
     return;
   }
-  // channel / tensor parameters of the lane's channels
-  LaneParams<D, P> lp;
+  // channel / tensor parameters of the lane's channels, constant over the layer's rows
+  uint4 lmn[P], linv[P];
 #pragma unroll
   for (int p = 0; p < P; ++p) {
+    lmn[p] = linv[p] = make_uint4(0, 0, 0, 0);
     const int h = p * HPW + (int)rl.slot;
     const kvmi_rt_section s = (h < g.num_heads && section_of(L, h)) ? L.sections[1] : L.sections[0];
-    if (h >= g.num_heads || s.axis == 1) {
-#pragma unroll
-      for (int k = 0; k < E; ++k) lp.mn[p][k] = 0.0f, lp.inv[p][k] = 0.0f;
-      continue;
-    }
-    const uint64_t pi = s.axis == 0 ? (uint64_t)(h - s.head_start) * D + rl.sub * E : 0;
-    const uint16_t* pmn = reinterpret_cast<const uint16_t*>(aux + s.aux_min_offset) + pi;
-    const uint16_t* pinv = reinterpret_cast<const uint16_t*>(aux + half + s.aux_scale_offset) + pi;
+    if (h >= g.num_heads || s.axis == 1) continue;
+    const uint16_t* pmn = reinterpret_cast<const uint16_t*>(aux + s.aux_min_offset);
+    const uint16_t* pinv = reinterpret_cast<const uint16_t*>(aux + half + s.aux_scale_offset);
     if (s.axis == 0) {
-      ld_seg<E>(pmn, lp.mn[p], true);
-      ld_seg<E>(pinv, lp.inv[p], true);
+      const uint64_t pi = (uint64_t)(h - s.head_start) * D + rl.sub * E;
+      lmn[p] = ld_seg(pmn + pi, true);
+      linv[p] = ld_seg(pinv + pi, true);
     } else {
-      const float a = ld_bf16(pmn), b = ld_bf16(pinv);
-#pragma unroll
-      for (int k = 0; k < E; ++k) lp.mn[p][k] = a, lp.inv[p][k] = b;
+      const uint32_t a = gld(pmn) * 0x10001u, b = gld(pinv) * 0x10001u;
+      lmn[p] = make_uint4(a, a, a, a);
+      linv[p] = make_uint4(b, b, b, b);
     }
   }
   const bool tok0 = L.num_sections > 0 && L.sections[0].axis == 1;
@@ -833,6 +810,8 @@ __global__ __launch_bounds__(kRtThreads) void rt_row_encode_kernel(kvmi_rt_geome
   for (int j = 0; j < R; ++j) {
     if ((uint32_t)j >= n) break;
     const uint64_t row = row0 + j;
+    float v[P][E];
+    transform_row<D, P>(g, c, rl, raw[j], v, scale);
     // token-axis statistics of the row, per section (two named sections: a local
     // array indexed by a run-time section number would live in scratch memory)
     QP tp0 = {}, tp1 = {};
@@ -844,7 +823,7 @@ __global__ __launch_bounds__(kRtThreads) void rt_row_encode_kernel(kvmi_rt_geome
         if (h >= g.num_heads) continue;
         float a = INFINITY, b = -INFINITY;
 #pragma unroll
-        for (int k = 0; k < E; ++k) a = fminf(a, v[j][p][k]), b = fmaxf(b, v[j][p][k]);
+        for (int k = 0; k < E; ++k) a = fminf(a, v[p][k]), b = fmaxf(b, v[p][k]);
         if (section_of(L, h)) {
           tmin1 = fminf(tmin1, a), tmax1 = fmaxf(tmax1, b);
         } else {
@@ -860,32 +839,29 @@ __global__ __launch_bounds__(kRtThreads) void rt_row_encode_kernel(kvmi_rt_geome
         if (rl.lane == (uint32_t)j) put_params(aux, half, L.sections[1], row, tp1);
       }
     }
-    uint8_t* out = packed + L.u8_offset + row * cols + rl.sub * E;
+    uint8_t* out = packed + L.u8_offset + row * cols;
 #pragma unroll
     for (int p = 0; p < P; ++p) {
       const int h = p * HPW + (int)rl.slot;
       if (h >= g.num_heads) continue;
       const bool second = section_of(L, h);
-      const kvmi_rt_section s = second ? L.sections[1] : L.sections[0];
-      const bool token = s.axis == 1;
-      const QP& t = second ? tp1 : tp0;
-      const float top = (float)(s.levels - 1);
-      uint32_t w[(E + 3) / 4];
+      const float top = (float)((second ? L.sections[1] : L.sections[0]).levels - 1);
+      float mn[E], inv[E];
+      unpack_seg(lmn[p], mn);
+      unpack_seg(linv[p], inv);
+      if (tok0 || tok1) {
+        const bool token = second ? tok1 : tok0;
+        const QP& t = second ? tp1 : tp0;
 #pragma unroll
-      for (int i = 0; i < (E + 3) / 4; ++i) w[i] = 0;
-#pragma unroll
-      for (int k = 0; k < E; k += 2) {
-        float a = v[j][p][k] - (token ? t.mn : lp.mn[p][k]);
-        float b = v[j][p][k + 1] - (token ? t.mn : lp.mn[p][k + 1]);
-        rn2(a, b);
-        a *= token ? t.inv : lp.inv[p][k];
-        b *= token ? t.inv : lp.inv[p][k + 1];
-        rn2(a, b);
-        a = fminf(fmaxf(rintf(a), 0.0f), top);
-        b = fminf(fmaxf(rintf(b), 0.0f), top);
-        w[k / 4] |= ((uint32_t)a | ((uint32_t)b << 8)) << (8 * (k % 4));
+        for (int k = 0; k < E; ++k) mn[k] = token ? t.mn : mn[k], inv[k] = token ? t.inv : inv[k];
       }
-      st_sym<E>(out + (int64_t)h * D, w);
+      uint32_t w[2] = {0, 0};
+#pragma unroll
+      for (int k = 0; k < E; ++k) {
+        const float q = __builtin_rintf(rn1(rn1(v[p][k] - mn[k]) * inv[k]));
+        w[k / 4] = __builtin_amdgcn_cvt_pk_u8_f32(__builtin_amdgcn_fmed3f(q, 0.0f, top), k % 4, w[k / 4]);
+      }
+      gst(reinterpret_cast<uint2*>(out + ((uint32_t)h * D + rl.sub * E)), make_uint2(w[0], w[1]));
     }
   }
 }
@@ -897,9 +873,9 @@ __global__ __launch_bounds__(kRtThreads) void rt_row_decode_kernel(kvmi_rt_geome
                                                                    const int64_t* __restrict__ block_ids, uint64_t rows,
                                                                    uint32_t num_layers, const uint8_t* __restrict__ packed,
                                                                    const uint8_t* __restrict__ aux, bool vec, float scale) {
-  constexpr int E = RowGeo<D>::E, HPW = RowGeo<D>::HPW, R = rows_per_wave<P>();
+  constexpr int HPW = RowGeo<D>::HPW, R = rows_per_wave<P>();
   const uint32_t nrows = (uint32_t)rows, groups = (nrows + R - 1) / R;
-  const uint32_t task = blockIdx.x * kRtWaves + (threadIdx.x >> 6);
+  const uint32_t task = blockIdx.x * kRtWaves + wave_index();
   if (task >= groups * num_layers) return;  // wave-uniform
   const uint32_t layer = task / groups;
   const uint32_t row0 = (task - layer * groups) * R;
@@ -908,113 +884,88 @@ __global__ __launch_bounds__(kRtThreads) void rt_row_decode_kernel(kvmi_rt_geome
   const RowLane rl = row_lane<D>();
   const uint64_t cols = (uint64_t)g.num_heads * D;
   const bool quant = g.flags & KVMI_RT_QUANTIZE;
-  LayerLanes<D, P> c;
-  layer_lanes<D, P>(g, L, rl, c);
-  const RowRef ref = row_ref(g, block_ids, row0, n, rl.lane);
-  float v[R][P][E];
-  if (!quant) {
+  // symbols (or bf16 rows) of all rows first, then the parameters
+  uint2 sym[R][P];
+  uint4 raw[R][P];
 #pragma unroll
-    for (int j = 0; j < R; ++j)
-#pragma unroll
-      for (int p = 0; p < P; ++p) {
-        const int h = p * HPW + (int)rl.slot;
-        if ((uint32_t)j < n && h < g.num_heads) {
-          ld_seg<E>(reinterpret_cast<const uint16_t*>(packed) + L.u8_offset + (row0 + j) * cols + (uint64_t)h * D +
-                        rl.sub * E, v[j][p], true);
-        } else {
-#pragma unroll
-          for (int k = 0; k < E; ++k) v[j][p][k] = 0.0f;
-        }
-      }
-  } else {
-    // symbols of all rows first, then the parameters
-    uint32_t w[R][P][(E + 3) / 4];
-#pragma unroll
-    for (int j = 0; j < R; ++j)
-#pragma unroll
-      for (int p = 0; p < P; ++p) {
-        const int h = p * HPW + (int)rl.slot;
-        if ((uint32_t)j < n && h < g.num_heads) {
-          ld_sym<E>(packed + L.u8_offset + (row0 + j) * cols + (uint64_t)h * D + rl.sub * E, w[j][p]);
-        } else {
-#pragma unroll
-          for (int i = 0; i < (E + 3) / 4; ++i) w[j][p][i] = 0;
-        }
-      }
-    // token parameters: lane j holds row row0 + j's (min, scale) of each section
-    float tmn0 = 0.0f, tsc0 = 0.0f, tmn1 = 0.0f, tsc1 = 0.0f;
-    if (rl.lane < n) {
-      if (L.num_sections > 0 && L.sections[0].axis == 1) {
-        tmn0 = ld_bf16(reinterpret_cast<const uint16_t*>(aux + L.sections[0].aux_min_offset) + row0 + rl.lane);
-        tsc0 = ld_bf16(reinterpret_cast<const uint16_t*>(aux + L.sections[0].aux_scale_offset) + row0 + rl.lane);
-      }
-      if (L.num_sections > 1 && L.sections[1].axis == 1) {
-        tmn1 = ld_bf16(reinterpret_cast<const uint16_t*>(aux + L.sections[1].aux_min_offset) + row0 + rl.lane);
-        tsc1 = ld_bf16(reinterpret_cast<const uint16_t*>(aux + L.sections[1].aux_scale_offset) + row0 + rl.lane);
-      }
-    }
+  for (int j = 0; j < R; ++j)
 #pragma unroll
     for (int p = 0; p < P; ++p) {
       const int h = p * HPW + (int)rl.slot;
-      const bool live = h < g.num_heads;
-      const bool second = live && section_of(L, h);
-      const kvmi_rt_section s = second ? L.sections[1] : L.sections[0];
-      float mn[E], sc[E];
-      if (live && s.axis != 1) {
-        const uint64_t pi = s.axis == 0 ? (uint64_t)(h - s.head_start) * D + rl.sub * E : 0;
-        const uint16_t* pmn = reinterpret_cast<const uint16_t*>(aux + s.aux_min_offset) + pi;
-        const uint16_t* psc = reinterpret_cast<const uint16_t*>(aux + s.aux_scale_offset) + pi;
-        if (s.axis == 0) {
-          ld_seg<E>(pmn, mn, true);
-          ld_seg<E>(psc, sc, true);
-        } else {
-          const float a = ld_bf16(pmn), b = ld_bf16(psc);
-#pragma unroll
-          for (int k = 0; k < E; ++k) mn[k] = a, sc[k] = b;
-        }
-      }
-#pragma unroll
-      for (int j = 0; j < R; ++j) {
-        // row j's parameters of both sections from lane j, then this lane's section
-        const float m0 = __shfl(tmn0, j, 64), m1 = __shfl(tmn1, j, 64);
-        const float s0 = __shfl(tsc0, j, 64), s1 = __shfl(tsc1, j, 64);
-        const float rmn = second ? m1 : m0, rsc = second ? s1 : s0;
-#pragma unroll
-        for (int k = 0; k < E; k += 2) {
-          const bool tok = live && s.axis == 1;
-          float a = (float)((w[j][p][k / 4] >> (8 * (k % 4))) & 0xffu) * (tok ? rsc : sc[k]);
-          float b = (float)((w[j][p][k / 4] >> (8 * (k % 4) + 8)) & 0xffu) * (tok ? rsc : sc[k + 1]);
-          rn2(a, b);
-          a += tok ? rmn : mn[k];
-          b += tok ? rmn : mn[k + 1];
-          rn2(a, b);
-          v[j][p][k] = a;
-          v[j][p][k + 1] = b;
-        }
-      }
+      const uint64_t at = L.u8_offset + (row0 + j) * cols;
+      const uint32_t in_row = (uint32_t)h * D + rl.sub * E;
+      sym[j][p] = make_uint2(0, 0);
+      raw[j][p] = make_uint4(0, 0, 0, 0);
+      if ((uint32_t)j >= n || h >= g.num_heads) continue;
+      if (quant) sym[j][p] = gld(reinterpret_cast<const uint2*>(packed + at + in_row));
+      else raw[j][p] = ld_seg(reinterpret_cast<const uint16_t*>(packed) + at + in_row, true);
+    }
+  LayerLanes<D, P> c;
+  layer_lanes<D, P>(g, L, rl, c);
+  const int64_t ref = row_ref(g, L, block_ids, row0, n, rl.lane);
+  // token parameters: lane j holds row row0 + j's (min, scale) of each section, packed
+  const bool tok0 = quant && L.num_sections > 0 && L.sections[0].axis == 1;
+  const bool tok1 = quant && L.num_sections > 1 && L.sections[1].axis == 1;
+  uint32_t t0 = 0, t1 = 0;
+  if (rl.lane < n) {
+    if (tok0) {
+      t0 = (uint32_t)gld(reinterpret_cast<const uint16_t*>(aux + L.sections[0].aux_min_offset) + row0 + rl.lane) |
+           (uint32_t)gld(reinterpret_cast<const uint16_t*>(aux + L.sections[0].aux_scale_offset) + row0 + rl.lane) << 16;
+    }
+    if (tok1) {
+      t1 = (uint32_t)gld(reinterpret_cast<const uint16_t*>(aux + L.sections[1].aux_min_offset) + row0 + rl.lane) |
+           (uint32_t)gld(reinterpret_cast<const uint16_t*>(aux + L.sections[1].aux_scale_offset) + row0 + rl.lane) << 16;
     }
   }
-  if (g.flags & KVMI_RT_TRANSFORM) {
+  uint4 lmn[P], lsc[P];
 #pragma unroll
-    for (int j = 0; j < R; ++j) fwht_rows<D, P>(v[j], rl.lane, scale);
+  for (int p = 0; p < P; ++p) {
+    lmn[p] = lsc[p] = make_uint4(0, 0, 0, 0);
+    const int h = p * HPW + (int)rl.slot;
+    if (!quant || h >= g.num_heads) continue;
+    const kvmi_rt_section s = section_of(L, h) ? L.sections[1] : L.sections[0];
+    if (s.axis == 1) continue;
+    const uint16_t* pmn = reinterpret_cast<const uint16_t*>(aux + s.aux_min_offset);
+    const uint16_t* psc = reinterpret_cast<const uint16_t*>(aux + s.aux_scale_offset);
+    if (s.axis == 0) {
+      const uint64_t pi = (uint64_t)(h - s.head_start) * D + rl.sub * E;
+      lmn[p] = ld_seg(pmn + pi, true);
+      lsc[p] = ld_seg(psc + pi, true);
+    } else {
+      const uint32_t a = gld(pmn) * 0x10001u, b = gld(psc) * 0x10001u;
+      lmn[p] = make_uint4(a, a, a, a);
+      lsc[p] = make_uint4(b, b, b, b);
+    }
   }
-  const uint16_t* signs = static_cast<const uint16_t*>(L.signs);
-  uint16_t* base = static_cast<uint16_t*>(L.cache) + L.channel_offset + rl.sub * E;
+  uint16_t* cache = static_cast<uint16_t*>(L.cache) + L.channel_offset;
 #pragma unroll
   for (int j = 0; j < R; ++j) {
     if ((uint32_t)j >= n) break;
-    const int64_t pb = __shfl(ref.pb, j, 64);
-    const uint32_t tok = (uint32_t)__shfl((int)ref.tok, j, 64);
-    uint16_t* row = base + pb * L.block_stride + (int64_t)tok * L.token_stride;
+    const uint32_t r0 = (uint32_t)__builtin_amdgcn_readlane((int)t0, j), r1 = (uint32_t)__builtin_amdgcn_readlane((int)t1, j);
+    uint16_t* out = cache + row_at(ref, j);
 #pragma unroll
     for (int p = 0; p < P; ++p) {
-      if (c.hc[p] < 0) continue;
-      if (signs) {
+      float v[E];
+      if (quant) {
+        float mn[E], sc[E];
+        unpack_seg(lmn[p], mn);
+        unpack_seg(lsc[p], sc);
+        if (tok0 || tok1) {
+          const bool second = section_of(L, p * HPW + (int)rl.slot), token = second ? tok1 : tok0;
+          const float rmn = bf_lo(second ? r1 : r0), rsc = bf_hi(second ? r1 : r0);
+#pragma unroll
+          for (int k = 0; k < E; ++k) mn[k] = token ? rmn : mn[k], sc[k] = token ? rsc : sc[k];
+        }
+        const uint32_t w[2] = {sym[j][p].x, sym[j][p].y};
 #pragma unroll
         for (int k = 0; k < E; ++k)
-          v[j][p][k] = __uint_as_float(__float_as_uint(v[j][p][k]) ^ (__float_as_uint(c.sg[p][k]) & 0x80000000u));
+          v[k] = rn1(rn1((float)((w[k / 4] >> (8 * (k % 4))) & 0xffu) * sc[k]) + mn[k]);
+      } else {
+        unpack_seg(raw[j][p], v);
       }
-      st_seg<E>(row + (int64_t)c.hc[p] * L.head_stride, v[j][p], vec);
+      if (g.flags & KVMI_RT_TRANSFORM) fwht_seg<D>(v, rl.sub, scale);
+      if (c.hc[p] < 0) continue;
+      st_seg(out + (c.hc[p] * L.head_stride + rl.sub * E), xor_seg(pack_seg(v), c.flip[p]), vec);
     }
   }
 }
@@ -1047,7 +998,6 @@ bool rt_row_head_dim(int D) { return D >= 8 && D <= 256; }
 // and row; wider rows take the generic path
 int rt_row_passes(int D, int H) {
   if (!rt_row_head_dim(D)) return 0;
-  int E = D <= 8 ? D : (D / 64 > 8 ? D / 64 : 8);
   const int hpw = 64 / (D / E);
   const int need = (H + hpw - 1) / hpw;
   int P = 1;
@@ -1122,8 +1072,14 @@ extern "C" int kvmi_rt_encode(const kvmi_rt_geometry* geom, const kvmi_rt_layer*
         float* partial = static_cast<float*>(canon);
         hipLaunchKernelGGL((rt_stats_kernel<D, PP>), dim3(wpl * (uint32_t)num_layers), dim3(kRtThreads), 0, s, g,
                            layers, block_ids, rows, partial, wpl, vec, scale);
-        hipLaunchKernelGGL(rt_stats_reduce_kernel, dim3((uint32_t)num_layers), dim3(kRtThreads), 0, s, g, layers,
-                           (const float*)partial, wpl, aux, half);
+        if (g.axes & 4u) {
+          hipLaunchKernelGGL(rt_stats_reduce_kernel, dim3((uint32_t)num_layers), dim3(kRtThreads), 0, s, g, layers,
+                             (const float*)partial, wpl, aux, half);
+        } else {
+          const uint32_t col_wgs = ((uint32_t)g.num_heads * D + 63) / 64;
+          hipLaunchKernelGGL(rt_stats_channel_kernel, dim3(col_wgs * (uint32_t)num_layers), dim3(kRtThreads), 0, s, g,
+                             layers, (const float*)partial, wpl, col_wgs, aux, half);
+        }
       }
       constexpr int R = rows_per_wave<PP>();
       const uint64_t tasks = (rows + R - 1) / R * (uint64_t)num_layers;
