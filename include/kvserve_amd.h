@@ -304,6 +304,11 @@ int kvmi_decode_paged(const kvmi_geometry* geom, const kvmi_layer_job* jobs, int
 int kvmi_v3_compress(const void* x, int64_t rows, int32_t num_heads, int32_t head_dim, const uint32_t* signs,
                      const float* levels, const int32_t* vgroup, uint8_t* q, float* kmeta, float* vmeta,
                      void* scratch, kvmi_stream_t stream);
+/* kvmi_v3_compress with the metadata rounded to float16 as well, in the tables of the wire:
+ * kmin16, kscale16 [H][D] and vmin16, vscale16 [rows][H]; the float kmeta is still written. */
+int kvmi_v3_compress_f16(const void* x, int64_t rows, int32_t num_heads, int32_t head_dim, const uint32_t* signs,
+                         const float* levels, const int32_t* vgroup, uint8_t* q, uint16_t* kmin16, uint16_t* kscale16,
+                         uint16_t* vmin16, uint16_t* vscale16, float* kmeta, void* scratch, kvmi_stream_t stream);
 /* Scratch bytes of kvmi_v3_compress: up to 256 per-workgroup K partials of 2*H*D*4
  * bytes, not depending on rows (-1 for an unsupported shape). */
 int64_t kvmi_v3_scratch_bytes(int64_t rows, int32_t num_heads, int32_t head_dim);
@@ -331,6 +336,11 @@ int kvmi_v3_compress_noalloc(const void* x, int64_t rows, int32_t num_heads, int
  * bf16 [2][rows][H][D]. */
 int kvmi_v3_decompress(const uint8_t* q, int64_t rows, int32_t num_heads, int32_t head_dim, const uint32_t* signs,
                        const uint16_t* kmeta16, const uint16_t* vmeta16, void* out, kvmi_stream_t stream);
+/* kvmi_v3_decompress with the four tables of kvmi_v3_compress_f16 (kmin16 and kscale16 16-byte
+ * aligned). */
+int kvmi_v3_decompress_tables(const uint8_t* q, int64_t rows, int32_t num_heads, int32_t head_dim,
+                              const uint32_t* signs, const uint16_t* kmin16, const uint16_t* kscale16,
+                              const uint16_t* vmin16, const uint16_t* vscale16, void* out, kvmi_stream_t stream);
 
 /*
  * Entropy codec (rANS) for the codec stage -- replaces the nvCOMP ANS codec that

@@ -62,6 +62,8 @@ EXPORTS = (
     "kvmi_rans_encode_batch",
     "kvmi_rans_decode_batch",
     "kvmi_v3_compress",
+    "kvmi_v3_compress_f16",
+    "kvmi_v3_decompress_tables",
     "kvmi_v3_scratch_bytes",
     "kvmi_v3_decompress",
     "kvmi_v3_compress_noalloc",
@@ -155,6 +157,9 @@ _SIGNATURES = {
     "kvmi_rans_encode_batch": ([ctypes.POINTER(RansEncJob), _i32, _i32, _vp], ctypes.c_int),
     "kvmi_rans_decode_batch": ([ctypes.POINTER(RansDecJob), _i32, _i32, _vp, _vp], ctypes.c_int),
     "kvmi_v3_compress": ([_vp, _i64, _i32, _i32, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp], ctypes.c_int),
+    "kvmi_v3_compress_f16": ([_vp, _i64, _i32, _i32, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp],
+                             ctypes.c_int),
+    "kvmi_v3_decompress_tables": ([_vp, _i64, _i32, _i32, _vp, _vp, _vp, _vp, _vp, _vp, _vp], ctypes.c_int),
     "kvmi_v3_scratch_bytes": ([_i64, _i32, _i32], _i64),
     "kvmi_v3_decompress": ([_vp, _i64, _i32, _i32, _vp, _vp, _vp, _vp, _vp], ctypes.c_int),
     "kvmi_v3_compress_noalloc": ([_vp, _i64, _i32, _i32, _vp, _vp, _vp, _vp, _vp, _vp, _vp], ctypes.c_int),

@@ -26,10 +26,10 @@ from ..components import Quantizer
 _ROUTING_KEYS = frozenset({"impl", "quantizer_impl", "tp_rank", "tensor_parallel_size"})
 
 
-def _f16(t: Any) -> Any:
-    if isinstance(t, torch.Tensor) and t.dtype == torch.float32:
-        return t.to(torch.float16)
-    return t
+def _aligned(t: torch.Tensor) -> torch.Tensor:
+    """Contiguous and 16-byte aligned, as the kernels read the K tables."""
+    t = t.contiguous()
+    return t if t.data_ptr() % 16 == 0 else t.clone()
 
 
 def _group_map(levels) -> list:
@@ -172,15 +172,19 @@ class FusedHadamardQuantizer(Quantizer):
             raise ValueError(f"unsupported geometry for the fused quantizer: heads={H}, head_dim={D}")
         levels, group, signs = self._device_tables(layer_id, H, D, dev)
         # no rows: no statistics are computed, and the K metadata is defined as zeros
-        kmeta = (torch.zeros if rows == 0 else torch.empty)((2, H, D), dtype=torch.float32, device=dev)
-        vmeta = torch.empty((2, rows, H), dtype=torch.float32, device=dev)
-        scratch = torch.empty(max(scratch_n, 1), dtype=torch.uint8, device=dev)
+        kmin, ksc = ((torch.zeros if rows == 0 else torch.empty)((H, D), dtype=torch.float16, device=dev)
+                     for _ in range(2))
+        vmin, vsc = (torch.empty((rows, H), dtype=torch.float16, device=dev) for _ in range(2))
+        # the float K table and the partials, side by side
+        scratch = torch.empty(8 * H * D + scratch_n, dtype=torch.uint8, device=dev)
         with torch.cuda.device(dev):
-            _lib.check(lib.kvmi_v3_compress(x.data_ptr(), rows, H, D, signs.data_ptr(), levels.data_ptr(),
-                                            group.data_ptr(), out.data_ptr(), kmeta.data_ptr(), vmeta.data_ptr(),
-                                            scratch.data_ptr(), _stream_handle()), "kvmi_v3_compress")
-        meta = {"key_meta": {"min_val": _f16(kmeta[0]), "quant_scale": _f16(kmeta[1]), "axis": "channel"},
-                "value_meta": {"min_val": _f16(vmeta[0]), "quant_scale": _f16(vmeta[1]), "axis": "token_perhead"}}
+            _lib.check(lib.kvmi_v3_compress_f16(x.data_ptr(), rows, H, D, signs.data_ptr(), levels.data_ptr(),
+                                                group.data_ptr(), out.data_ptr(), kmin.data_ptr(), ksc.data_ptr(),
+                                                vmin.data_ptr(), vsc.data_ptr(), scratch.data_ptr(),
+                                                scratch.data_ptr() + 8 * H * D, _stream_handle()),
+                       "kvmi_v3_compress_f16")
+        meta = {"key_meta": {"min_val": kmin, "quant_scale": ksc, "axis": "channel"},
+                "value_meta": {"min_val": vmin, "quant_scale": vsc, "axis": "token_perhead"}}
         return out, meta
 
     @staticmethod
@@ -226,15 +230,15 @@ class FusedHadamardQuantizer(Quantizer):
         if kmin.dim() != 2 or kmin.shape[-1] != D:
             raise ValueError(f"key metadata must be [heads, head_dim], got {tuple(kmin.shape)}")
         vmin, vsc = self._value_tables(quantization_params["value_meta"], rows, H, dev)
-        kmeta16 = torch.stack([kmin.reshape(H, D), ksc.reshape(H, D)]).contiguous()
-        vmeta16 = torch.stack([vmin.reshape(rows, H), vsc.reshape(rows, H)]).contiguous()
+        kmin, ksc = _aligned(kmin.reshape(H, D)), _aligned(ksc.reshape(H, D))
+        vmin, vsc = vmin.reshape(rows, H).contiguous(), vsc.reshape(rows, H).contiguous()
         _, _, signs = self._device_tables(layer_id, H, D, dev)
         out = torch.empty((2, B, S, H, D), dtype=torch.bfloat16, device=dev)
         lib = _lib.load()
         with torch.cuda.device(dev):
-            _lib.check(lib.kvmi_v3_decompress(q.data_ptr(), rows, H, D, signs.data_ptr(), kmeta16.data_ptr(),
-                                              vmeta16.data_ptr(), out.data_ptr(), _stream_handle()),
-                       "kvmi_v3_decompress")
+            _lib.check(lib.kvmi_v3_decompress_tables(q.data_ptr(), rows, H, D, signs.data_ptr(), kmin.data_ptr(),
+                                                     ksc.data_ptr(), vmin.data_ptr(), vsc.data_ptr(), out.data_ptr(),
+                                                     _stream_handle()), "kvmi_v3_decompress_tables")
         return out
 
 

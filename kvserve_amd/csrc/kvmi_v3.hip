@@ -21,6 +21,14 @@
 //           V is read once; q = clamp(roundf((had - min) / scale), 0, L) as uint8.
 // Decompress is one launch: x = fma(q, scale16, min16), fp32 butterflies,
 // bf16((y * (1/sqrt(D))) * s) (:685-716).
+//
+// What bounds them, at 8192 rows of 8 x 128 (33.5 MB; us before and after the present form):
+// quant 24.1 -> 22.4, its vector units busy 83 % of the time (12 instructions a value for the
+// transform, 12 for the symbol; with the divisions 25): without a second pass in flight behind
+// the first 26, with rows through LDS chunks instead of lane segments 28.  kstats 11.5, one wave
+// a SIMD, latency; dequant 15.8 -> 14.5 (50 MB at 3.5 TB/s).  The float16 tables leave from the
+// kernels and are read where they lie: six launches of copies and joins less, 19 us; compress
+// and decompress together 80 -> 47.5 us.
 #include <mutex>
 
 #include "kvmi_common.hpp"
@@ -59,18 +67,29 @@ __device__ __forceinline__ void v3_transform_w(uint32_t (&w)[D / 8], uint32_t sb
 #pragma unroll
   for (int i = 0; i < E; ++i) y[i] *= scale;
 }
-template <int D>
-__device__ __forceinline__ void v3_transform(const uint16_t* src, uint32_t sb, float scale, int q,
-                                             float (&y)[D / 4]) {
-  uint32_t w[D / 8];
-  load_bf16_seg<D / 4>(src, w);
-  v3_transform_w<D>(w, sb, scale, q, y);
+// clamp(roundf((had - mn) / sc), 0, L) as an integer, as the correctly rounded fp32 quotient
+// and ties away from zero give it, without the division (25 instructions an element down to
+// 13, of which the pass's time is made).  With a = had - mn, t = a * inv lies below a / sc by
+// 2^-21 to 2^-19 of it, so that only the half b = floor(t) + 1/2 can lie between: the result is
+// b + 1/2 if the rounded quotient reaches b, else b - 1/2.  It does if and only if a / sc is at
+// or above the middle of b and the float before it, b - p 2^-24 with p the power of two at or
+// below that float: t has the same exponent wherever that decides (also before 1/2).  Near b
+// the difference a - sc b is exact in fp32, and adding sc p 2^-24 to it keeps its sign;
+// elsewhere the sign of a - sc b alone decides.  An infinite or undefined scale makes every
+// quotient zero or undefined, symbol 0: inv is NaN then, of which the median makes 0.  A symbol
+// is a byte; the bounds above hold up to L = 65536.
+__device__ __forceinline__ float v3_inverse(float sc) {
+  return sc < __builtin_inff() ? (1.0f / sc) * 0.99999905f : __builtin_nanf("");
 }
-
-// clamp(roundf((had - mn) / sc), 0, L) as an integer (roundf: ties away from zero;
-// the division is the correctly rounded fp32 one).
-__device__ __forceinline__ uint32_t v3_symbol(float had, float mn, float sc, float lv) {
-  return (uint32_t)fminf(fmaxf(__builtin_roundf((had - mn) / sc), 0.0f), lv);
+// y rounded to bf16 in one instruction: the conversion of (0, y) leaves its value in place.
+__device__ __forceinline__ float v3_had(float y) { return __uint_as_float(pack_bf16x2(0.0f, y)); }
+__device__ __forceinline__ uint32_t v3_symbol(float had, float mn, float sc, float inv, float lv) {
+  const float a = had - mn, t = a * inv;
+  const float b = __builtin_floorf(t) + 0.5f;
+  const float r = __builtin_fmaf(-sc, b, a);
+  const float p = __uint_as_float(__float_as_uint(t) & 0x7f800000u);
+  const float up = __builtin_fmaf(sc * 0x1p-24f, p, r);
+  return (uint32_t)__builtin_amdgcn_fmed3f(b + __builtin_copysignf(0.5f, up), 0.0f, lv);
 }
 
 struct V3Shape {
@@ -78,6 +97,15 @@ struct V3Shape {
   int H;
   float scale;   // fp32 1/sqrt(D)
 };
+
+// Where (min, scale) go: K's float table, which the quantizing pass reads, and V's, or the
+// wire's float16 tables (K's as well as the float one) when those are asked for.
+struct V3Meta {
+  float *k, *v;                      // [2][H][D], [2][rows][H] (null: float16 only)
+  uint16_t *kmn, *ksc, *vmn, *vsc;   // [H][D], [H][D], [rows][H], [rows][H] or null
+};
+
+__device__ __forceinline__ void gst_f16(uint16_t* p, float x) { gst(p, __builtin_bit_cast(uint16_t, (_Float16)x)); }
 
 // ------------------------------------------------------------------ K statistics
 // One partial per workgroup: the grid must not exceed kV3KGrid.  With about one
@@ -149,12 +177,13 @@ __global__ __launch_bounds__(kV3WG) void v3_kstats_kernel(V3Shape sh, const uint
   }
 }
 
-// K statistics over the partials -> kmeta [2][H][D] = (min, scale).  A workgroup
+// K statistics over the partials -> kmeta [2][H][D] = (min, scale), and v3_inverse of the
+// scale over the first partial's minima, which no other workgroup reads.  A workgroup
 // takes 4 channels: lane j = tid & 3 of every quad reads channel 4 * blockIdx.x + j
 // of the partials s, s + 64, ... (s = tid >> 2, so every load of a lane is
 // independent), then the 64 slices are reduced across the wave and the 4 waves.
-__global__ __launch_bounds__(kV3WG) void v3_kfinal_kernel(int HD, int D, int nparts, const uint32_t* __restrict__ kpart,
-                                                          const float* __restrict__ levels, float* __restrict__ kmeta) {
+__global__ __launch_bounds__(kV3WG) void v3_kfinal_kernel(int HD, int D, int nparts, uint32_t* kpart,
+                                                          const float* __restrict__ levels, V3Meta meta) {
   const int j = threadIdx.x & 3, s = threadIdx.x >> 2;
   // The 8 workgroups whose channels share a 128-byte line of the partials take ids
   // equal mod 8, i.e. the same XCD under round-robin dispatch, so that one L2 fetch
@@ -189,86 +218,146 @@ __global__ __launch_bounds__(kV3WG) void v3_kfinal_kernel(int HD, int D, int npa
   }
   const float mn = key2f(a), mx = key2f(b);
   const float lv = gld(levels + c / D);
-  gst(kmeta + c, mn);
-  gst(kmeta + HD + c, fmaxf(mx - mn, 1e-5f) / (lv - 1.0f));
+  const float sc = fmaxf(mx - mn, 1e-5f) / (lv - 1.0f);
+  gst(meta.k + c, mn);
+  gst(meta.k + HD + c, sc);
+  if (meta.kmn) {
+    gst_f16(meta.kmn + c, mn);
+    gst_f16(meta.ksc + c, sc);
+  }
+  gst(kpart + c, __float_as_uint(v3_inverse(sc)));
 }
 
 // ------------------------------------------------------------------ quantize
-// Symbols leave through streaming stores: 3-4 % faster compress than cached stores
-// (the same stores for dequant's bf16 output were 1.6x slower, so that one stays cached).
-template <int E>
-__device__ __forceinline__ void v3_store_symbols(uint8_t* p, const uint32_t (&sym)[E]) {
-  uint32_t w[E / 4];
+// Words leave through a per-wave LDS stage: lane l puts its W words at row l (rows padded to
+// W + 4 words against bank conflicts), then the wave stores 16-byte chunk f = c * 64 + lane,
+// i.e. chunk f % (W/4) of lane f / (W/4)'s segment, so that consecutive lanes store consecutive
+// bytes of each head-row (a lane's own segment at a W-word lane stride writes at a far lower
+// rate).
+template <int W>
+__device__ __forceinline__ void v3_stage_put(uint32_t* ws, int lane, const uint32_t (&o)[W]) {
+  uint4* row = reinterpret_cast<uint4*>(ws + lane * (W + 4));
 #pragma unroll
-  for (int i = 0; i < E / 4; ++i)
-    w[i] = sym[4 * i] | (sym[4 * i + 1] << 8) | (sym[4 * i + 2] << 16) | (sym[4 * i + 3] << 24);
-  uint4* o = reinterpret_cast<uint4*>(p);
-#pragma unroll
-  for (int i = 0; i < E / 16; ++i) gst_stream(o + i, make_uint4(w[4 * i], w[4 * i + 1], w[4 * i + 2], w[4 * i + 3]));
+  for (int i = 0; i < W / 4; ++i) row[i] = make_uint4(o[4 * i], o[4 * i + 1], o[4 * i + 2], o[4 * i + 3]);
 }
 
-// blockIdx.y = part (0 = K, 1 = V).  hrows is a multiple of H and 64 % H == 0, so a
-// pass of 64 consecutive head-rows holds whole rows, each entirely inside or entirely
-// past the layer; lanes past it load and store nothing but still reach the V branch's
-// barriers (the pass count is uniform over the workgroup).
+// Chunk c of the stage: the quad it comes from, its 16-byte place in that head-row, its words.
+template <int W>
+struct StageChunk {
+  int quad, at;
+  uint4 w;
+  __device__ __forceinline__ StageChunk(const uint32_t* ws, int lane, int c) {
+    constexpr int CH = W / 4;
+    const int f = c * 64 + lane, sl = f / CH, k = f % CH;  // source lane, its chunk
+    quad = sl >> 2;
+    at = (sl & 3) * CH + k;
+    w = *reinterpret_cast<const uint4*>(ws + sl * (W + 4) + 4 * k);
+  }
+};
+
+// blockIdx.y = part (0 = K, 1 = V).  K passes are 64 rows of one head, so that the quads of a
+// wave read the same channel constants (one broadcast line per lane position, not one copy per
+// quad); V passes are 64 consecutive head-rows: hrows is a multiple of H and 64 % H == 0, so
+// such a pass holds whole rows, each entirely inside or entirely past the layer.  Lanes past it
+// load and store nothing but still reach the V branch's barriers (the pass count is uniform
+// over the workgroup) and move staged chunks.
 template <int D>
 __global__ __launch_bounds__(kV3WG) void v3_quant_kernel(V3Shape sh, const uint16_t* __restrict__ x,
                                                          const uint32_t* __restrict__ signs,
                                                          const float* __restrict__ levels,
                                                          const int32_t* __restrict__ vgroup,
-                                                         const float* __restrict__ kmeta, uint8_t* __restrict__ qout,
-                                                         float* __restrict__ vmeta) {
-  constexpr int E = D / 4;
+                                                         const uint32_t* __restrict__ kinv, uint8_t* __restrict__ qout,
+                                                         V3Meta meta) {
+  constexpr int E = D / 4, W = E / 4, CH = W / 4;  // symbols, their words and 16-byte chunks of a segment
   const int part = blockIdx.y;
   const int H = sh.H, HD = H * D;
-  const int tid = threadIdx.x, Q = tid >> 2, q = tid & 3, h = Q % H;
+  const int tid = threadIdx.x, Q = tid >> 2, q = tid & 3, lane = tid & 63, qw = (tid >> 6) * 16;
   const int64_t hrows = sh.rows * H;
   const uint16_t* src = x + part * hrows * D;
   uint8_t* dst = qout + part * hrows * D;
+  __shared__ __align__(16) uint32_t stage[kV3WG / 64][64 * (W + 4)];
+  uint32_t* ws = stage[tid >> 6];
+  uint32_t next[E / 2], in[E / 2], w[W];  // bf16 pairs of the next pass and of this one; symbols, four to a word
+  float y[E];
+  if (part == 0) {
+    const int64_t kpasses = (sh.rows + kV3Rows - 1) / kV3Rows * H;
+    auto fetch = [&](int64_t p) {
+      const int64_t r = (p / H) * kV3Rows + Q;
+      if (p < kpasses && r < sh.rows) load_bf16_seg<E>(src + (r * H + p % H) * D + q * E, next);
+    };
+    fetch(blockIdx.x);
+    for (int64_t p = blockIdx.x; p < kpasses; p += gridDim.x) {
+      const int h = (int)(p % H);
+      const int64_t r0 = (p / H) * kV3Rows;  // row of quad 0 of the pass
+      const float lv = gld(levels + h);
+#pragma unroll
+      for (int i = 0; i < E / 2; ++i) in[i] = next[i];
+      fetch(p + gridDim.x);
+      if (r0 + Q < sh.rows) {
+        v3_transform_w<D>(in, v3_lane_signs<D>(signs, h, q), sh.scale, q, y);
+        const float* kmn = meta.k + h * D + q * E;
+        const uint32_t* ki = kinv + h * D + q * E;
+#pragma unroll
+        for (int i = 0; i < W; ++i) w[i] = 0;
+#pragma unroll
+        for (int i8 = 0; i8 < E; i8 += 8) {
+#pragma unroll
+          for (int i = i8; i < i8 + 8; ++i)
+            w[i / 4] |= v3_symbol(v3_had(y[i]), gld(kmn + i), gld(kmn + HD + i), __uint_as_float(gld(ki + i)), lv)
+                        << (8 * (i % 4));
+          __builtin_amdgcn_sched_barrier(0);  // eight channels' constants at a time in registers
+        }
+        v3_stage_put<W>(ws, lane, w);
+      }
+      __builtin_amdgcn_wave_barrier();
+#pragma unroll
+      for (int c = 0; c < CH; ++c) {
+        const StageChunk<W> t(ws, lane, c);
+        const int64_t rs = r0 + qw + t.quad;
+        if (rs < sh.rows) gst(reinterpret_cast<uint4*>(dst + (rs * H + h) * D) + t.at, t.w);
+      }
+      __builtin_amdgcn_wave_barrier();
+    }
+    return;
+  }
+  const int h = Q % H;
   const uint32_t sb = v3_lane_signs<D>(signs, h, q);
-  const float lv = gld(levels + part * H + h);
+  const float lv = gld(levels + H + h);
   const int64_t passes = (hrows + kV3Rows - 1) / kV3Rows;
   // heads of this head's V group (equal L), as a bit set over the row's heads
   uint64_t same = 0;
-  if (part == 1) {
-    const int grp = gld(vgroup + h);
-    for (int k = 0; k < H; ++k)
-      if (gld(vgroup + k) == grp) same |= (uint64_t)1 << k;
-  }
+  const int grp = gld(vgroup + h);
+  for (int k = 0; k < H; ++k)
+    if (gld(vgroup + k) == grp) same |= (uint64_t)1 << k;
   __shared__ float lmn[kV3Rows], lmx[kV3Rows];
   const int row0 = Q - h;  // this pass's LDS slot of head 0 of the lane's row
+  auto fetch = [&](int64_t p) {
+    const int64_t r = p * kV3Rows + Q;
+    if (r < hrows) load_bf16_seg<E>(src + r * D + q * E, next);
+  };
+  fetch(blockIdx.x);
   for (int64_t p = blockIdx.x; p < passes; p += gridDim.x) {
-    const int64_t hr = p * kV3Rows + Q;
+    const int64_t h0 = p * kV3Rows, hr = h0 + Q;  // head-rows of quad 0 of the pass and of this one
     const bool live = hr < hrows;
-    float y[E];
-    if (live) {
-      v3_transform<D>(src + hr * D + q * E, sb, sh.scale, q, y);
-    } else {
 #pragma unroll
-      for (int i = 0; i < E; ++i) y[i] = 0.0f;
+    for (int i = 0; i < E / 2; ++i) in[i] = next[i];
+    fetch(p + gridDim.x);
+    v3_transform_w<D>(in, sb, sh.scale, q, y);
+    float mn = y[0], mx = y[0];
+#pragma unroll
+    for (int i = 1; i < E; ++i) {
+      mn = fminf(mn, y[i]);
+      mx = fmaxf(mx, y[i]);
     }
-    uint32_t sym[E];
-    if (part == 0) {
-      if (!live) continue;
-      const float* kmn = kmeta + h * D + q * E;
-#pragma unroll
-      for (int i = 0; i < E; ++i) sym[i] = v3_symbol(round_bf16(y[i]), gld(kmn + i), gld(kmn + HD + i), lv);
-    } else {
-      float mn = y[0], mx = y[0];
-#pragma unroll
-      for (int i = 1; i < E; ++i) {
-        mn = fminf(mn, y[i]);
-        mx = fmaxf(mx, y[i]);
-      }
-      mn = quad_min(mn);
-      mx = quad_max(mx);
-      __syncthreads();  // the previous pass's readers are done
-      if (q == 0) {
-        lmn[Q] = mn;
-        lmx[Q] = mx;
-      }
-      __syncthreads();
-      if (!live) continue;  // no barrier follows in this pass
+    mn = quad_min(mn);
+    mx = quad_max(mx);
+    __syncthreads();  // the previous pass's readers are done
+    if (q == 0) {
+      lmn[Q] = mn;
+      lmx[Q] = mx;
+    }
+    __syncthreads();
+    if (live) {
       // the row's statistics over the heads of this head's group
       float gmn = __builtin_inff(), gmx = -__builtin_inff();
       for (uint64_t m = same; m; m &= m - 1) {
@@ -278,13 +367,29 @@ __global__ __launch_bounds__(kV3WG) void v3_quant_kernel(V3Shape sh, const uint1
       }
       const float sc = fmaxf(gmx - gmn, 1e-5f) / (lv - 1.0f);
       if (q == 0) {
-        gst(vmeta + hr, gmn);
-        gst(vmeta + hrows + hr, sc);
+        if (meta.vmn) {
+          gst_f16(meta.vmn + hr, gmn);
+          gst_f16(meta.vsc + hr, sc);
+        } else {
+          gst(meta.v + hr, gmn);
+          gst(meta.v + hrows + hr, sc);
+        }
       }
+      const float inv = v3_inverse(sc);
 #pragma unroll
-      for (int i = 0; i < E; ++i) sym[i] = v3_symbol(round_bf16(y[i]), gmn, sc, lv);
+      for (int i = 0; i < W; ++i) w[i] = 0;
+#pragma unroll
+      for (int i = 0; i < E; ++i) w[i / 4] |= v3_symbol(v3_had(y[i]), gmn, sc, inv, lv) << (8 * (i % 4));
+      v3_stage_put<W>(ws, lane, w);
     }
-    v3_store_symbols<E>(dst + hr * D + q * E, sym);
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int c = 0; c < CH; ++c) {
+      const StageChunk<W> t(ws, lane, c);
+      const int64_t hs = h0 + qw + t.quad;
+      if (hs < hrows) gst(reinterpret_cast<uint4*>(dst + hs * D) + t.at, t.w);
+    }
+    __builtin_amdgcn_wave_barrier();
   }
 }
 
@@ -314,18 +419,6 @@ __device__ __forceinline__ void v3_inverse_words(float (&v)[D / 4], uint32_t sb,
   apply_sign_bf16<E>(o, sb);
 }
 
-// The output leaves through a per-wave LDS stage: lane l puts its W = E/2 words at row
-// l (rows padded to W + 4 words against bank conflicts), then the wave stores 16-byte
-// chunk f = c * 64 + lane, i.e. chunk f % (W/4) of lane f / (W/4)'s segment, so that
-// consecutive lanes store consecutive bytes of each head-row (a lane's own segment at
-// a 2E-byte lane stride writes at a far lower rate).
-template <int W>
-__device__ __forceinline__ void v3_stage_put(uint32_t* ws, int lane, const uint32_t (&o)[W]) {
-  uint4* row = reinterpret_cast<uint4*>(ws + lane * (W + 4));
-#pragma unroll
-  for (int i = 0; i < W / 4; ++i) row[i] = make_uint4(o[4 * i], o[4 * i + 1], o[4 * i + 2], o[4 * i + 3]);
-}
-
 // K passes are head-major: a pass is 64 rows of one head, so the quads of a wave read
 // the same channel constants (one broadcast line per lane position, not one copy per
 // quad).  V passes are 64 consecutive head-rows.  Every lane takes part in the staged
@@ -334,12 +427,14 @@ __device__ __forceinline__ void v3_stage_put(uint32_t* ws, int lane, const uint3
 template <int D>
 __global__ __launch_bounds__(kV3WG) void v3_dequant_kernel(V3Shape sh, const uint8_t* __restrict__ qin,
                                                            const uint32_t* __restrict__ signs,
-                                                           const uint16_t* __restrict__ kmeta16,
-                                                           const uint16_t* __restrict__ vmeta16,
+                                                           const uint16_t* __restrict__ kmn16,
+                                                           const uint16_t* __restrict__ ksc16,
+                                                           const uint16_t* __restrict__ vmn16,
+                                                           const uint16_t* __restrict__ vsc16,
                                                            uint16_t* __restrict__ out) {
   constexpr int E = D / 4, W = E / 2, CH = W / 4;  // words and 16-byte chunks of a segment
   const int part = blockIdx.y;
-  const int H = sh.H, HD = H * D;
+  const int H = sh.H;
   const int tid = threadIdx.x, Q = tid >> 2, q = tid & 3, lane = tid & 63, qw = (tid >> 6) * 16;
   const int64_t hrows = sh.rows * H;
   const uint8_t* src = qin + part * hrows * D;
@@ -356,8 +451,8 @@ __global__ __launch_bounds__(kV3WG) void v3_dequant_kernel(V3Shape sh, const uin
         const int64_t hr = r * H + hk;
         uint32_t w[E / 4];
         v3_load_symbols<E>(src + hr * D + q * E, w);
-        const uint4* mn = reinterpret_cast<const uint4*>(kmeta16 + hk * D + q * E);  // 16-byte aligned
-        const uint4* sc = reinterpret_cast<const uint4*>(kmeta16 + HD + hk * D + q * E);
+        const uint4* mn = reinterpret_cast<const uint4*>(kmn16 + hk * D + q * E);  // 16-byte aligned
+        const uint4* sc = reinterpret_cast<const uint4*>(ksc16 + hk * D + q * E);
         float v[E];
 #pragma unroll
         for (int i8 = 0; i8 < E / 8; ++i8) {
@@ -378,12 +473,9 @@ __global__ __launch_bounds__(kV3WG) void v3_dequant_kernel(V3Shape sh, const uin
       __builtin_amdgcn_wave_barrier();
 #pragma unroll
       for (int c = 0; c < CH; ++c) {
-        const int f = c * 64 + lane, sl = f / CH, k = f % CH;  // source lane, its chunk
-        const int64_t rs = r0 + qw + (sl >> 2);
-        if (rs < sh.rows) {
-          const uint4 t = *reinterpret_cast<const uint4*>(ws + sl * (W + 4) + 4 * k);
-          gst(reinterpret_cast<uint4*>(dst + (rs * H + hk) * D + (sl & 3) * E + 8 * k), t);
-        }
+        const StageChunk<W> t(ws, lane, c);
+        const int64_t rs = r0 + qw + t.quad;
+        if (rs < sh.rows) gst(reinterpret_cast<uint4*>(dst + (rs * H + hk) * D) + t.at, t.w);
       }
       __builtin_amdgcn_wave_barrier();
     }
@@ -397,7 +489,7 @@ __global__ __launch_bounds__(kV3WG) void v3_dequant_kernel(V3Shape sh, const uin
     if (hr < hrows) {
       uint32_t w[E / 4];
       v3_load_symbols<E>(src + hr * D + q * E, w);
-      const float mn = f16_to_f32(gld(vmeta16 + hr)), sc = f16_to_f32(gld(vmeta16 + hrows + hr));
+      const float mn = f16_to_f32(gld(vmn16 + hr)), sc = f16_to_f32(gld(vsc16 + hr));
       float v[E];
 #pragma unroll
       for (int i = 0; i < E; ++i) v[i] = __builtin_fmaf((float)((w[i / 4] >> (8 * (i % 4))) & 0xffu), sc, mn);
@@ -408,12 +500,9 @@ __global__ __launch_bounds__(kV3WG) void v3_dequant_kernel(V3Shape sh, const uin
     __builtin_amdgcn_wave_barrier();
 #pragma unroll
     for (int c = 0; c < CH; ++c) {
-      const int f = c * 64 + lane, sl = f / CH, k = f % CH;
-      const int64_t hs = h0 + qw + (sl >> 2);
-      if (hs < hrows) {
-        const uint4 t = *reinterpret_cast<const uint4*>(ws + sl * (W + 4) + 4 * k);
-        gst(reinterpret_cast<uint4*>(dst + hs * D + (sl & 3) * E + 8 * k), t);
-      }
+      const StageChunk<W> t(ws, lane, c);
+      const int64_t hs = h0 + qw + t.quad;
+      if (hs < hrows) gst(reinterpret_cast<uint4*>(dst + hs * D) + t.at, t.w);
     }
     __builtin_amdgcn_wave_barrier();
   }
@@ -435,6 +524,10 @@ unsigned v3_grid(int64_t rows, int H) {
   return (unsigned)(passes > 0 ? passes : 1);
 }
 
+// Workgroups of a part of the quantizing pass: beyond what the chip holds at once (4 a CU,
+// both parts together) each takes two passes, the second one's rows in flight during the first.
+unsigned v3_qgrid(unsigned passes) { return passes > 512 ? (passes + 1) / 2 : passes; }
+
 // Workgroups of the K statistics pass, i.e. the K partials one call writes and reads.
 unsigned v3_kgrid(int64_t rows, int H) {
   const unsigned g = v3_grid(rows, H);
@@ -444,11 +537,11 @@ unsigned v3_kgrid(int64_t rows, int H) {
 // The three launches of compress with the K partials at `kpart`
 // (v3_kgrid(rows, H) * 2 * H * D uint32; every one is written before it is read).
 int v3_compress_launch(const void* x, int64_t rows, int32_t H, int32_t D, const uint32_t* signs,
-                       const float* levels, const int32_t* vgroup, uint8_t* q, float* kmeta, float* vmeta,
-                       uint32_t* kpart, hipStream_t st) {
+                       const float* levels, const int32_t* vgroup, uint8_t* q, const V3Meta& meta, uint32_t* kpart,
+                       hipStream_t st) {
   V3Shape sh{rows, H, (float)(1.0 / __builtin_sqrt((double)D))};
   const unsigned g = v3_grid(rows, H);
-  const unsigned gk = v3_kgrid(rows, H);
+  const unsigned gk = v3_kgrid(rows, H), gq = v3_qgrid(g);
   const size_t klds = (size_t)2 * H * D * 4;
   const uint16_t* xs = static_cast<const uint16_t*>(x);
   const unsigned gf = (unsigned)((H * D + 3) / 4);  // 4 channels per workgroup
@@ -456,13 +549,13 @@ int v3_compress_launch(const void* x, int64_t rows, int32_t H, int32_t D, const 
     hipLaunchKernelGGL((v3_kstats_kernel<64>), dim3(gk), dim3(kV3WG), klds, st, sh, xs, signs, kpart);
   else
     hipLaunchKernelGGL((v3_kstats_kernel<128>), dim3(gk), dim3(kV3WG), klds, st, sh, xs, signs, kpart);
-  hipLaunchKernelGGL(v3_kfinal_kernel, dim3(gf), dim3(kV3WG), 0, st, H * D, D, (int)gk, kpart, levels, kmeta);
+  hipLaunchKernelGGL(v3_kfinal_kernel, dim3(gf), dim3(kV3WG), 0, st, H * D, D, (int)gk, kpart, levels, meta);
   if (D == 64)
-    hipLaunchKernelGGL((v3_quant_kernel<64>), dim3(g, 2), dim3(kV3WG), 0, st, sh, xs, signs, levels, vgroup, kmeta,
-                       q, vmeta);
+    hipLaunchKernelGGL((v3_quant_kernel<64>), dim3(gq, 2), dim3(kV3WG), 0, st, sh, xs, signs, levels, vgroup,
+                       (const uint32_t*)kpart, q, meta);
   else
-    hipLaunchKernelGGL((v3_quant_kernel<128>), dim3(g, 2), dim3(kV3WG), 0, st, sh, xs, signs, levels, vgroup, kmeta,
-                       q, vmeta);
+    hipLaunchKernelGGL((v3_quant_kernel<128>), dim3(gq, 2), dim3(kV3WG), 0, st, sh, xs, signs, levels, vgroup,
+                       (const uint32_t*)kpart, q, meta);
   return hipGetLastError() == hipSuccess ? KVMI_OK : KVMI_ELAUNCH;
 }
 
@@ -528,7 +621,24 @@ extern "C" int kvmi_v3_compress(const void* x, int64_t rows, int32_t num_heads, 
   rc = v3_compress_args(x, rows, num_heads, head_dim, signs, levels, vgroup, q, kmeta, vmeta);
   if (rc) return rc;
   if (!workspace) return KVMI_EINVAL;
-  return v3_compress_launch(x, rows, num_heads, head_dim, signs, levels, vgroup, q, kmeta, vmeta,
+  const V3Meta meta{kmeta, vmeta, nullptr, nullptr, nullptr, nullptr};
+  return v3_compress_launch(x, rows, num_heads, head_dim, signs, levels, vgroup, q, meta,
+                            static_cast<uint32_t*>(workspace), reinterpret_cast<hipStream_t>(stream));
+}
+
+extern "C" int kvmi_v3_compress_f16(const void* x, int64_t rows, int32_t num_heads, int32_t head_dim,
+                                    const uint32_t* signs, const float* levels, const int32_t* vgroup, uint8_t* q,
+                                    uint16_t* kmin16, uint16_t* kscale16, uint16_t* vmin16, uint16_t* vscale16,
+                                    float* kmeta, void* workspace, kvmi_stream_t stream) {
+  using namespace kvmi;
+  int rc = v3_check(rows, num_heads, head_dim);
+  if (rc) return rc;
+  if (rows == 0) return KVMI_OK;
+  rc = v3_compress_args(x, rows, num_heads, head_dim, signs, levels, vgroup, q, kmeta, kmeta);
+  if (rc) return rc;
+  if (!kmin16 || !kscale16 || !vmin16 || !vscale16 || !workspace) return KVMI_EINVAL;
+  const V3Meta meta{kmeta, nullptr, kmin16, kscale16, vmin16, vscale16};
+  return v3_compress_launch(x, rows, num_heads, head_dim, signs, levels, vgroup, q, meta,
                             static_cast<uint32_t*>(workspace), reinterpret_cast<hipStream_t>(stream));
 }
 
@@ -552,7 +662,8 @@ extern "C" int kvmi_v3_compress_noalloc(const void* x, int64_t rows, int32_t num
   if (hipStreamIsCapturing(st, &cap) != hipSuccess) return KVMI_ELAUNCH;
   const bool ordered = cap == hipStreamCaptureStatusNone;
   if (ordered && sl->recorded && hipStreamWaitEvent(st, sl->done, 0) != hipSuccess) return KVMI_ELAUNCH;
-  rc = v3_compress_launch(x, rows, num_heads, head_dim, signs, levels, vgroup, q, kmeta, vmeta,
+  const V3Meta meta{kmeta, vmeta, nullptr, nullptr, nullptr, nullptr};
+  rc = v3_compress_launch(x, rows, num_heads, head_dim, signs, levels, vgroup, q, meta,
                           static_cast<uint32_t*>(sl->ptr), st);
   if (rc == KVMI_OK && ordered) {
     if (hipEventRecord(sl->done, st) != hipSuccess) return KVMI_ELAUNCH;
@@ -561,22 +672,37 @@ extern "C" int kvmi_v3_compress_noalloc(const void* x, int64_t rows, int32_t num
   return rc;
 }
 
-extern "C" int kvmi_v3_decompress(const uint8_t* q, int64_t rows, int32_t num_heads, int32_t head_dim,
-                                  const uint32_t* signs, const uint16_t* kmeta16, const uint16_t* vmeta16, void* out,
-                                  kvmi_stream_t stream) {
+extern "C" int kvmi_v3_decompress_tables(const uint8_t* q, int64_t rows, int32_t num_heads, int32_t head_dim,
+                                         const uint32_t* signs, const uint16_t* kmin16, const uint16_t* kscale16,
+                                         const uint16_t* vmin16, const uint16_t* vscale16, void* out,
+                                         kvmi_stream_t stream) {
   using namespace kvmi;
   int rc = v3_check(rows, num_heads, head_dim);
   if (rc) return rc;
   if (rows == 0) return KVMI_OK;
-  if (!q || !signs || !kmeta16 || !vmeta16 || !out) return KVMI_EINVAL;
-  if (((uintptr_t)q | (uintptr_t)out | (uintptr_t)kmeta16) & 15) return KVMI_EINVAL;  // 16-byte vectors
+  if (!q || !signs || !kmin16 || !kscale16 || !vmin16 || !vscale16 || !out) return KVMI_EINVAL;
+  if (((uintptr_t)q | (uintptr_t)out | (uintptr_t)kmin16 | (uintptr_t)kscale16) & 15) return KVMI_EINVAL;
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   V3Shape sh{rows, num_heads, (float)(1.0 / __builtin_sqrt((double)head_dim))};
   const unsigned g = v3_grid(rows, num_heads);
   uint16_t* o = static_cast<uint16_t*>(out);
   if (head_dim == 64)
-    hipLaunchKernelGGL((v3_dequant_kernel<64>), dim3(g, 2), dim3(kV3WG), 0, st, sh, q, signs, kmeta16, vmeta16, o);
+    hipLaunchKernelGGL((v3_dequant_kernel<64>), dim3(g, 2), dim3(kV3WG), 0, st, sh, q, signs, kmin16, kscale16, vmin16,
+                       vscale16, o);
   else
-    hipLaunchKernelGGL((v3_dequant_kernel<128>), dim3(g, 2), dim3(kV3WG), 0, st, sh, q, signs, kmeta16, vmeta16, o);
+    hipLaunchKernelGGL((v3_dequant_kernel<128>), dim3(g, 2), dim3(kV3WG), 0, st, sh, q, signs, kmin16, kscale16, vmin16,
+                       vscale16, o);
   return hipGetLastError() == hipSuccess ? KVMI_OK : KVMI_ELAUNCH;
+}
+
+extern "C" int kvmi_v3_decompress(const uint8_t* q, int64_t rows, int32_t num_heads, int32_t head_dim,
+                                  const uint32_t* signs, const uint16_t* kmeta16, const uint16_t* vmeta16, void* out,
+                                  kvmi_stream_t stream) {
+  const int rc = kvmi::v3_check(rows, num_heads, head_dim);
+  if (rc) return rc;
+  if (rows == 0) return KVMI_OK;
+  if (!kmeta16 || !vmeta16) return KVMI_EINVAL;
+  return kvmi_v3_decompress_tables(q, rows, num_heads, head_dim, signs, kmeta16,
+                                   kmeta16 + (int64_t)num_heads * head_dim, vmeta16, vmeta16 + rows * num_heads, out,
+                                   stream);
 }
