@@ -546,7 +546,7 @@ class Plan:
         if codec.transform:
             self.signs = SIGNS.table(codec.seed, packet.layer_ids, codec.H, codec.D, dev)
         self.prof = codec._profile_table(packet.profiles, dev)
-        self.keys = codec._kstats_scratch(L, dev)
+        self.keys = codec._kstats_scratch(L, dev) if kind == "compress" else None  # statistics only
         self.jobs = codec._jobs(pools, ids, packet.streams, packet.chunks, packet.kmeta, packet.vmeta,
                                 self.signs, self.prof, self.keys, B)
         # a device block table is checked by the first launch of the plan's first run
