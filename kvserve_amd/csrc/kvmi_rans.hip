@@ -514,25 +514,26 @@ __device__ __forceinline__ void ring_ahead(RingFeed& f, uint32_t lane) {
   f.ahead = u < f.units ? gld(f.region + u / 2) : 0u;
 }
 
-// Stages the next kRefill units of the word region unless `want` units (or all) are staged.
+// Stages the word region kRefill units at a time until `want` units (or all) are staged.
 __device__ __forceinline__ void ring_fill(uint16_t* ring, RingFeed& f, uint32_t want, uint32_t lane) {
-  if (f.filled >= want || f.filled >= f.units) return;
-  const uint32_t at = f.filled & (kRing - 1);
-  reinterpret_cast<uint32_t*>(ring + at)[lane] = f.ahead;
-  if (at == 0 && 2u * lane < kMirror) reinterpret_cast<uint32_t*>(ring + kRing)[lane] = f.ahead;
-  f.filled += kRefill;
-  ring_ahead(f, lane);
-  wave_lds_fence();
+  while (f.filled < want && f.filled < f.units) {
+    const uint32_t at = f.filled & (kRing - 1);
+    reinterpret_cast<uint32_t*>(ring + at)[lane] = f.ahead;
+    if (at == 0 && 2u * lane < kMirror) reinterpret_cast<uint32_t*>(ring + kRing)[lane] = f.ahead;
+    f.filled += kRefill;
+    ring_ahead(f, lane);
+    wave_lds_fence();
+  }
 }
 
 // Steps 0..255 of one sub-block (block runs run0 .. run0 + 7); returns the final
 // state.  Before each group of kGroup steps (at most 64 * kGroup words) the ring holds at
-// least that many unread units: a group reads no more than one refill brings, so one is
-// enough.  It starts only while fewer than 64 * kGroup units are staged past q, and kRing >=
-// 64 * kGroup + kRefill, so it overwrites only units below q.
+// least that many unread units: one refill brings as many as a group reads, and the first
+// group, whose words may begin at unit 1, takes two.  A refill starts only while fewer than
+// 64 * kGroup units are staged past q, and kRing >= 64 * kGroup + kRefill, so it overwrites
+// only units below q.
 constexpr uint32_t kGroup = 2;
 static_assert(kRing >= kGroup * kLanes + kRefill, "ring too small for the refill policy");
-static_assert(kRefill >= kGroup * kLanes, "one refill serves a group");
 
 // Decode table: slot -> symbol, frequency and the slot's offset in its symbol's range (bits
 // 20..31); a step is one LDS read off the state.  Up to 7 bits the symbol has bits 0..6 and the

@@ -39,3 +39,22 @@ def test_every_kind_of_frequency(cuda, w, tail):
     st = ops.rans_encode(torch.from_numpy(body.copy()).to(cuda), s.size, w)
     assert np.array_equal(st.cpu().numpy(), ref)
     assert np.array_equal(ops.rans_decode(st, s.size, w).cpu().numpy(), body)
+
+
+@pytest.mark.parametrize("extra", [0, 4, 7])
+def test_first_two_steps_take_a_word_in_every_lane(cuda, extra):
+    """Symbols of frequency one at steps 0 and 1 of every lane of a sub-block, so that these steps
+    read 128 words, from unit 0 of the word region (an even count) or 1 (an odd one)."""
+    s = np.zeros(65536, np.uint8)
+    lanes = np.arange(64)
+    s[lanes * 32] = 1 + lanes
+    s[lanes * 32 + 1] = 65 + lanes
+    late = 5 * 2048 + 7 * 32 + 3
+    s[late : late + extra] = 200 + np.arange(extra)  # an odd number of further words in one lane
+    body = crans.pack(s, 8)
+    ref = crans.encode_packed(body, s.size, 8)
+    count = int(ref[40:44].view(np.uint32)[0]) >> 1
+    assert count >= 128 and count % 2 == (extra > 0)
+    st = ops.rans_encode(torch.from_numpy(body.copy()).to(cuda), s.size, 8)
+    assert np.array_equal(st.cpu().numpy(), ref)
+    assert np.array_equal(ops.rans_decode(st, s.size, 8).cpu().numpy(), body)
