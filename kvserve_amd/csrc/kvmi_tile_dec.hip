@@ -82,7 +82,6 @@ __global__ __launch_bounds__(kTileThreads, kDecOcc<D>) void tile_decode_kernel(G
 
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
   __shared__ TileTables T;
-  __shared__ int ok;
   uint32_t* smask = reinterpret_cast<uint32_t*>(lds);
   float2* kc = reinterpret_cast<float2*>(lds + a.off_tab);
   uint4* tb = reinterpret_cast<uint4*>(lds + a.off_wave + wave * a.wave_bytes);
@@ -129,23 +128,21 @@ __global__ __launch_bounds__(kTileThreads, kDecOcc<D>) void tile_decode_kernel(G
       d->w = x[u].w;
     }
   };
-  // the first image's loads are in flight during the table set-up
+  // The stream is as long as its header says, so nothing of it is read before the header
+  // matches: every wave checks for itself, while the loads of the first tables are in flight.
+  // The first image's loads are then in flight during the rest of the table set-up.
+  const bool ok = (g.flags & KVMI_F_NO_HEADER) || header_matches(job.stream, bits, job.chunk_symbols);
+  tile_stage_profile(T, job.profile, H);
+  if (TR) tile_signs<D>(smask, job.signs, H);
+  if (!ok) {  // the same for the whole workgroup
+    if (threadIdx.x == 0 && blockIdx.x == 0 && part0 == 0) atomicOr(err, KVMI_ERR_BAD_HEADER);
+    return;
+  }
   const int step = kTileWaves * a.ST;
   int st = tok0 + wave * a.ST;
   uint4 pk[kPackedRegs<D>];
   if (st < tok_end) fetch(part0, st, pk);
-  if (threadIdx.x == 0) {
-    int good = 1;
-    if (!(g.flags & KVMI_F_NO_HEADER)) {
-      good = header_matches(job.stream, bits, job.chunk_symbols);
-      if (!good && blockIdx.x == 0 && part0 == 0) atomicOr(err, KVMI_ERR_BAD_HEADER);
-    }
-    ok = good;
-  }
-  tile_stage_profile(T, job.profile, H);
-  if (TR) tile_signs<D>(smask, job.signs, H);
   __syncthreads();
-  if (!ok) return;
   tile_positions(T, H);
   const int tab1 = (a.tabs & 1) ? H * (D + 4) : 0;
   if ((a.tabs & 1) && part0 == 0) tile_consts<D, false>(kc, T, g, job.kmeta, 0);

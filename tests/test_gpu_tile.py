@@ -11,6 +11,7 @@ do the same arithmetic and have to agree bit for bit.
 import pytest
 import torch
 
+from kvserve_amd import _lib
 from kvserve_amd.engine import FusedKVCodec
 from kvserve_amd.profiles import section_profile, whole_layer_profile
 
@@ -136,3 +137,24 @@ def test_tile_special_values(case):
     x, y = (torch.nan_to_num(t.float(), nan=123.0, posinf=1e9, neginf=-1e9) for t in out)
     close = (x - y).abs() <= (y.abs() * 2.0 ** -7 if transform else 0.0)
     assert bool(close.all())
+
+
+@pytest.mark.parametrize("case", [(6, 96, 16, 8, "permuted", CT, True, 9), (8, 128, 16, 4, "native", ("token", "channel"), True, 33),
+                                  (8, 64, 16, 4, "permuted", CT, False, 40)], ids=lambda c: f"{c[0]}-{c[1]}-{c[3]}-{c[6]}")
+def test_tile_decode_reads_nothing_of_a_stream_whose_header_differs(case):
+    """A stream of 1-bit symbols, as long as its own header says, in the place of a wider one:
+    the error word is set, the caches keep their contents, and (by the order of the kernel's
+    reads) nothing behind the short stream is touched."""
+    H, D, S, bits, layout, axes, transform, B = case
+    gen = torch.Generator(device="cuda").manual_seed(6)
+    pools = _pools(case, gen, 2)
+    codec, plan = _run(case, pools, list(range(B)), _profiles(case, 2), "mfma")
+    narrow = FusedKVCodec(H, D, S, 1, 7, transform=transform, layout=layout, axes=axes, fwht="mfma")
+    short = narrow.compress(pools, list(range(B)), [whole_layer_profile(H, 2, 2)] * 2)
+    assert short.streams[0].numel() < plan.packet.streams[0].numel()
+    dst = [torch.full_like(p, 7.0) for p in pools]
+    back = codec.plan_decompress(plan.packet, dst, list(range(B)))
+    back.jobs[:, 2] = short.streams[0].data_ptr()
+    back.run()
+    assert back.error_code() == _lib.ERR_BAD_HEADER
+    assert all(bool((t == 7.0).all()) for t in dst)
