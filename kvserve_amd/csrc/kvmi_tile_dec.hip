@@ -195,12 +195,8 @@ __global__ __launch_bounds__(kTileThreads, kDecOcc<D>) void tile_decode_kernel(G
 #pragma unroll
             for (int p = 0; p < 4; ++p) {
               const float4 c = *reinterpret_cast<const float4*>(kd + 16 * s + 2 * p);
-              if constexpr (TR) {
-                const uint32_t spk = pack_bf16x2(sy[2 * p] * c.y, sy[2 * p + 1] * c.w);
-                w[p] = pack_bf16x2(add_lo(spk, c.x), add_hi(spk, c.z));
-              } else {  // an infinite scale stays in its own channel (see tile_diff)
-                w[p] = pack_bf16x2(rbf(sy[2 * p] * c.y) + c.x, rbf(sy[2 * p + 1] * c.w) + c.z);
-              }
+              // a product that is infinite stays in its own channel (see tile_diff)
+              w[p] = pack_bf16x2(rbf(sy[2 * p] * c.y) + c.x, rbf(sy[2 * p + 1] * c.w) + c.z);
             }
           } else {
 #pragma unroll

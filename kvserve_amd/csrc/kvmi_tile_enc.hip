@@ -76,17 +76,20 @@ __device__ __forceinline__ float clamp_level(float q, float lev) {
   return r;
 }
 
-// (bf16(m0 - lo(y)), bf16(m1 - hi(y))).  The dot products of rsub_rbf_pair multiply the
-// pair's other element by 0, so an infinity would reach its neighbour; behind a transform
-// both elements of a pair hold it anyway, without one it belongs to its own channel only.
-template <bool TR>
+// (bf16(m0 - lo(y)), bf16(m1 - hi(y))).  Not the dot products of rsub_rbf_pair: those multiply
+// the pair's other element by 0, so that an infinity would reach its neighbour, and behind a
+// transform too a sum may overflow in one channel alone.  Written out, because the compiler
+// unpacks the pairs of a whole tile at once and spills (D = 128: 108 bytes a lane, K per token
+// and V per channel of 16 x 4096 x 8 x 128 both ways 223 us against 201).
 __device__ __forceinline__ void tile_diff(uint32_t y, float m0, float m1, float& t0, float& t1) {
-  if constexpr (TR) {
-    rsub_rbf_pair(y, m0, m1, t0, t1);
-  } else {
-    t0 = rbf(m0 - bf_lo(y));
-    t1 = rbf(m1 - bf_hi(y));
-  }
+  asm("v_lshlrev_b32 %0, 16, %2\n\t"
+      "v_and_b32 %1, 0xffff0000, %2\n\t"
+      "v_sub_f32 %0, %3, %0\n\t"
+      "v_sub_f32 %1, %4, %1\n\t"
+      "v_cvt_pk_bf16_f32 %0, 0, %0\n\t"
+      "v_cvt_pk_bf16_f32 %1, 0, %1"
+      : "=&v"(t0), "=&v"(t1)
+      : "v"(y), "v"(m0), "v"(m1));
 }
 
 // Waves per SIMD the registers are limited to.
@@ -224,7 +227,7 @@ __global__ __launch_bounds__(kTileThreads, kEncOcc<D>) void tile_encode_kernel(G
             for (int i = 0; i < 16; i += 2) {
               const float4 c = *reinterpret_cast<const float4*>(kq + tail + 32 * cp + i);
               float t0, t1;
-              tile_diff<TR>(y[i / 2], c.x, c.z, t0, t1);
+              tile_diff(y[i / 2], c.x, c.z, t0, t1);
               q[i] = clamp_level(rbf(t0 * c.y), lev);
               q[i + 1] = clamp_level(rbf(t1 * c.w), lev);
             }
@@ -260,7 +263,7 @@ __global__ __launch_bounds__(kTileThreads, kEncOcc<D>) void tile_encode_kernel(G
 #pragma unroll
             for (int i = 0; i < 16; i += 2) {
               float t0, t1;
-              tile_diff<TR>(y[cp][i / 2], mn, mn, t0, t1);
+              tile_diff(y[cp][i / 2], mn, mn, t0, t1);
               q[i] = clamp_level(rbf(t0 * nrcp), lev);
               q[i + 1] = clamp_level(rbf(t1 * nrcp), lev);
             }

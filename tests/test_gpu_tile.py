@@ -13,7 +13,7 @@ import torch
 
 from kvserve_amd import _lib
 from kvserve_amd.engine import FusedKVCodec
-from kvserve_amd.profiles import section_profile, whole_layer_profile
+from kvserve_amd.profiles import rademacher_sign_bits, section_profile, whole_layer_profile
 
 pytestmark = pytest.mark.gpu
 
@@ -158,3 +158,51 @@ def test_tile_decode_reads_nothing_of_a_stream_whose_header_differs(case):
     back.run()
     assert back.error_code() == _lib.ERR_BAD_HEADER
     assert all(bool((t == 7.0).all()) for t in dst)
+
+
+@pytest.mark.parametrize("case", [(6, 96, 16, 4, "permuted", CT, True, 9), (5, 80, 16, 3, "permuted", ("token", "channel"), True, 20),
+                                  (8, 128, 16, 4, "native", ("channel", "channel"), True, 33)], ids=lambda c: f"{c[0]}-{c[1]}-{c[3]}")
+def test_tile_overflow_in_one_channel_leaves_its_neighbours(case):
+    """A finite row of 2^122 in the signs of one row of the transform: the sum of that channel
+    (2^128 over 64 channels) is infinite, every other channel of the row exactly 0.  Its symbols
+    and metadata are those of the row kernels, bit for bit, and so is the decoded row where a
+    scale's product overflows in one channel (an infinity of either sign, no NaN)."""
+    H, D, S, bits, layout, axes, transform, B = case
+    gen = torch.Generator(device="cuda").manual_seed(8)
+    pools = _pools(case, gen, 1)
+    chunk = 128 if D == 128 else 64
+    order = list(range(B))
+    profiles = [whole_layer_profile(H, TOP[bits], TOP[bits])]
+    signs = torch.from_numpy(rademacher_sign_bits(7, 0, H, D).view("int32")).cuda().to(torch.int64)
+    e = torch.arange(chunk, device="cuda")
+    for h, f in ((0, 6), (H - 1, 17)):
+        parity = sum((e & f) >> b & 1 for b in range(7)) & 1
+        flip = (signs[h, e // 32] >> (e % 32)) & 1
+        row = torch.where((parity ^ flip).bool(), -1.0, 1.0) * 2.0 ** (122 if chunk == 64 else 121)
+        pools[0][:, 3, 2, h] = 0.0
+        pools[0][:, 3, 2, h, :chunk] = row.to(torch.bfloat16)
+    tile, a = _run(case, pools, order, profiles, "mfma")
+    rows, b = _run(case, pools, order, profiles, "rows")
+    assert torch.isinf(b.packet.kmeta.float()).any() or torch.isinf(b.packet.vmeta.float()).any()
+    same = lambda x, y: torch.equal(torch.nan_to_num(x.float(), nan=123.0), torch.nan_to_num(y.float(), nan=123.0))  # noqa: E731
+    assert same(a.packet.kmeta, b.packet.kmeta) and same(a.packet.vmeta, b.packet.vmeta)
+    shape = (2, H, B * S, D) if layout == "permuted" else (2, B * S, H, D)
+    sym = [_unpack(p.packet.streams[0], bits).view(shape) for p in (a, b)]
+    if layout == "native":
+        sym = [s.permute(0, 2, 1, 3) for s in sym]
+    for h in (0, H - 1):
+        x, y = (s[:, h, 3 * S + 2] for s in sym)
+        assert torch.equal(x, y), (x, y)
+    # decode: one channel whose scale makes its product infinite from symbol 2 on
+    part = 0 if axes[0] == "channel" else 1
+    meta = (b.packet.kmeta, b.packet.vmeta)[part]
+    meta[:, 0], meta[:, 1] = 0.0, 1.0
+    meta[:, 1, :, 10] = 3e38
+    out = []
+    for codec in (tile, rows):
+        dst = [torch.zeros_like(pools[0])]
+        codec.plan_decompress(b.packet, dst, order).run()
+        out.append(dst[0][part, order].float())
+    x, y = out
+    assert torch.isinf(y).any() and torch.equal(torch.isinf(x), torch.isinf(y)) and torch.equal(torch.isnan(x), torch.isnan(y))
+    assert torch.equal(x[torch.isinf(y)], y[torch.isinf(y)])
