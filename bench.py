@@ -34,6 +34,7 @@ Hadamard quantizer (impl "tilelang_fused", kvmi_v3_*).
 from __future__ import annotations
 
 import argparse
+import ctypes
 import json
 import os
 import platform
@@ -106,9 +107,8 @@ CONNECTOR_PROFILE = {
 
 
 def hip_kernel_names(codec, S: int, H: int, D: int, bits: int, cplan=None) -> dict:
-    """Name of the HIP kernel each entry point runs for this geometry (MFMA, wave tiles for
-    what those do not take, or the register-FWHT kernels: quad-per-row or generic rows
-    where they are forced or nothing else serves the geometry)."""
+    """Name of the HIP kernel each entry point runs for this geometry: MFMA, or what
+    kvmi_paged_kernels says (wave tiles, quad-per-row or generic rows)."""
     default_axes = tuple(getattr(codec, "axes", ("channel", "token"))) == ("channel", "token")
     pow2 = D in (64, 128) and default_axes
     if D == 256 and H <= 16 and default_axes and codec.fwht == "mfma" and codec.transform:
@@ -134,21 +134,29 @@ def hip_kernel_names(codec, S: int, H: int, D: int, bits: int, cplan=None) -> di
         if cplan is not None and getattr(cplan, "workspace", None) is not None:  # the one-pass kernel runs
             names["kvmi_compress_paged"] = f"onepass_kernel<{D // 32}, {bits}, false>"
         return names
-    if codec.fwht == "valu" and pow2 and H <= 16 and 128 % H == 0:  # quad-per-row register FWHT
-        return {"kvmi_encode_paged": f"encode_kernel<{D}, {bits}>", "kvmi_decode_paged": f"decode_kernel<{D}, {bits}>",
-                "kvmi_kstats_paged": f"kstats_kernel<{D}>", "finalize": "kstats_finalize_kernel"}
+    from kvserve_amd import _lib
+
+    geo = _lib.Geometry(block_size=S, num_heads=H, head_dim=D, bits=bits, max_groups=1)
+    geo.flags = {"valu": _lib.F_VALU_FWHT, "rows": _lib.F_ROW_FWHT}.get(codec.fwht, 0)
+    geo.flags |= 0 if codec.transform else _lib.F_NO_TRANSFORM
+    geo.flags |= _lib.F_NATIVE_LAYOUT if getattr(codec, "layout", "permuted") == "native" else 0
+    geo.flags |= {"channel": 0, "token": _lib.F_K_TOKEN, "tensor": _lib.F_K_TENSOR}[codec.axes[0]]
+    geo.flags |= {"token": 0, "channel": _lib.F_V_CHANNEL, "tensor": _lib.F_V_TENSOR}[codec.axes[1]]
+    blocks = max(1, getattr(cplan, "max_blocks", 1))
     lpr = 1 << max(0, (D // 16 - 1).bit_length())  # generic rows: next_pow2(D / 16) lanes per row
-    rows = {"kvmi_encode_paged": f"rows_encode_kernel<{lpr}, {bits}>", "kvmi_decode_paged":
-            f"rows_decode_kernel<{lpr}, {bits}>", "kvmi_kstats_paged": f"rows_stats_kernel<{lpr}>",
-            "finalize": "rows_finalize_kernel"}
-    if codec.fwht != "mfma" or D not in (64, 80, 96, 112, 128, 160, 192, 224, 256) or H > 32:
-        return rows
-    tr = "true" if codec.transform else "false"  # wave tiles, where the workgroup's LDS allows (tile_eligible)
-    w = 4 if bits == 4 else 0
-    return {"kvmi_encode_paged": f"tile_encode_kernel<{D}, {tr}, {w}>",
-            "kvmi_decode_paged": f"tile_decode_kernel<{D}, {tr}, {w}>",
-            "kvmi_kstats_paged": f"tile_stats_kernel<{D}>" if codec.transform else "tile_plain_stats_kernel",
-            "finalize": "rows_finalize_kernel"}
+    tile = f"{D}, {'true' if codec.transform else 'false'}, {4 if bits == 4 else 0}"
+    names = {}
+    for call, decode in (("kvmi_encode_paged", 0), ("kvmi_decode_paged", 1)):
+        family = _lib.load().kvmi_paged_kernels(ctypes.byref(geo), 1, blocks, decode, None)
+        kind = "decode" if decode else "encode"
+        names[call] = {_lib.KERNELS_TILE: f"tile_{kind}_kernel<{tile}>", _lib.KERNELS_QUAD: f"{kind}_kernel<{D}, {bits}>",
+                       _lib.KERNELS_ROWS: f"rows_{kind}_kernel<{lpr}, {bits}>"}[family]
+        if not decode:
+            stats = f"tile_stats_kernel<{D}>" if codec.transform else "tile_plain_stats_kernel"
+            names["kvmi_kstats_paged"] = {_lib.KERNELS_TILE: stats, _lib.KERNELS_QUAD: f"kstats_kernel<{D}>",
+                                          _lib.KERNELS_ROWS: f"rows_stats_kernel<{lpr}>"}[family]
+            names["finalize"] = "kstats_finalize_kernel" if family == _lib.KERNELS_QUAD else "rows_finalize_kernel"
+    return names
 
 
 def compress_kernels(names: dict, cplan) -> list:

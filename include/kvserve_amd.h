@@ -82,13 +82,13 @@ typedef struct ihipStream_t* kvmi_stream_t;
 #define KVMI_F_TWO_PASS 32u     /* kvmi_compress_paged: statistics pass + encode pass (K read twice) */
 /* Quantization axes (quantizer_func.py:41-49; KVServeQuantizer axis_key / axis_value,
  * kvserve_quantizer.py:136-139).  Default (no flag): K per channel, V per token.  At most
- * one flag per part; any of them selects the generic row kernels. */
+ * one flag per part. */
 #define KVMI_F_K_TOKEN 64u    /* K statistics per token over the heads of a K group */
 #define KVMI_F_K_TENSOR 128u  /* one K statistic pair per K group */
 #define KVMI_F_V_CHANNEL 256u /* V statistics per channel of each head */
 #define KVMI_F_V_TENSOR 512u  /* one V statistic pair per V group */
 /* Force the generic row kernels (register FWHT with DPP exchanges over next_pow2(D)/16
- * lanes of a row) instead of MFMA or the quad-per-row kernels. */
+ * lanes of a row) instead of MFMA, wave tiles or the quad-per-row kernels. */
 #define KVMI_F_ROW_FWHT 1024u
 
 /* Launch-wide geometry shared by every job of one call. */
@@ -213,6 +213,20 @@ int kvmi_check_block_ids(kvmi_layer_job* jobs, int32_t num_jobs, int32_t* err, k
 int kvmi_hadamard(const void* in, void* out, int64_t rows, int32_t num_heads,
                   int32_t head_dim, const uint32_t* signs, int32_t inverse,
                   kvmi_stream_t stream);
+
+/*
+ * Which kernels a paged call of this geometry runs (host only, no counterpart in the
+ * reference): KVMI_KERNELS_* of kvmi_kstats_paged and kvmi_encode_paged (decode = 0) or of
+ * kvmi_decode_paged (decode = 1), or KVMI_EINVAL.  `shape` (may be NULL) receives int32[4],
+ * the launch shape of wave tiles: tokens of a tile, tiles of a wave's image, tokens of a
+ * workgroup's run, and the parts (K, V) a workgroup takes; zeros for the other kernels.
+ */
+#define KVMI_KERNELS_MFMA 0
+#define KVMI_KERNELS_TILE 1
+#define KVMI_KERNELS_QUAD 2
+#define KVMI_KERNELS_ROWS 3
+int kvmi_paged_kernels(const kvmi_geometry* geom, int32_t num_jobs, int32_t max_blocks, int32_t decode,
+                       int32_t* shape);
 
 /*
  * Pass 1 of compress: per-channel K statistics over all tokens of each job

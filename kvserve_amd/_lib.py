@@ -37,6 +37,8 @@ F_K_TENSOR = 128
 F_V_CHANNEL = 256
 F_V_TENSOR = 512
 F_ROW_FWHT = 1024
+# kvmi_paged_kernels
+KERNELS_MFMA, KERNELS_TILE, KERNELS_QUAD, KERNELS_ROWS = 0, 1, 2, 3
 
 # Every symbol include/kvserve_amd.h declares.
 EXPORTS = (
@@ -49,6 +51,7 @@ EXPORTS = (
     "kvmi_scatter_blocks_kv_adjacent",
     "kvmi_check_block_ids",
     "kvmi_hadamard",
+    "kvmi_paged_kernels",
     "kvmi_kstats_paged",
     "kvmi_encode_paged",
     "kvmi_decode_paged",
@@ -144,6 +147,7 @@ _SIGNATURES = {
     "kvmi_check_block_ids": ([_vp, _i32, _vp, _vp], ctypes.c_int),
     "kvmi_scatter_blocks_kv_adjacent": ([_vp, _vp, _i32, _i64, _vp, _vp], ctypes.c_int),
     "kvmi_hadamard": ([_vp, _vp, _i64, _i32, _i32, _vp, _i32, _vp], ctypes.c_int),
+    "kvmi_paged_kernels": ([ctypes.POINTER(Geometry), _i32, _i32, _i32, ctypes.POINTER(_i32)], ctypes.c_int),
     "kvmi_kstats_paged": ([ctypes.POINTER(Geometry), _vp, _i32, _i32, _vp, _vp], ctypes.c_int),
     "kvmi_encode_paged": ([ctypes.POINTER(Geometry), _vp, _i32, _i32, _vp, _vp], ctypes.c_int),
     "kvmi_decode_paged": ([ctypes.POINTER(Geometry), _vp, _i32, _i32, _vp, _vp], ctypes.c_int),

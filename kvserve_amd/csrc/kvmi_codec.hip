@@ -1,6 +1,6 @@
 // Fused paged compress / decompress kernels for gfx950, register FWHT, one quad of
 // lanes per row (D in {64, 128}, H dividing 128, H <= 16), run where the caller forces
-// them (KVMI_F_VALU_FWHT), and the entry points of the paged codec: the transform profile
+// them (KVMI_F_VALU_FWHT) or blocks are too small for the others, and the entry points of the paged codec: the transform profile
 // runs the MFMA kernels, what those do not take the wave tiles (kvmi_tile.hpp), the rest the
 // generic row kernels (kvmi_rows.hip); see the families in kvmi_common.hpp.
 //
@@ -412,6 +412,36 @@ void set_valu_bpw(Geo* g) {
 }  // namespace
 }  // namespace kvmi
 
+namespace kvmi {
+namespace {
+
+// The family a call runs (KVMI_KERNELS_*); `view` is the geometry the MFMA kernels are given
+// (head_dim 256 as paired heads).
+int paged_kernels(const Geo& g, int32_t max_blocks, bool decode, Geo* view) {
+  *view = g;
+  if (paired_view(g, view) || mfma_eligible(g)) return KVMI_KERNELS_MFMA;
+  if (tile_serves(g, max_blocks, decode)) return KVMI_KERNELS_TILE;
+  return quad_eligible(g) ? KVMI_KERNELS_QUAD : KVMI_KERNELS_ROWS;
+}
+
+}  // namespace
+}  // namespace kvmi
+
+extern "C" int kvmi_paged_kernels(const kvmi_geometry* geom, int32_t num_jobs, int32_t max_blocks, int32_t decode,
+                                  int32_t* shape) {
+  using namespace kvmi;
+  Geo g, v;
+  const int rc = check_geo(geom, num_jobs, max_blocks, &g);
+  if (rc) return rc;
+  const int family = paged_kernels(g, max_blocks, decode != 0, &v);
+  if (shape) {
+    int32_t out[4] = {0, 0, 0, 0};
+    if (family == KVMI_KERNELS_TILE && num_jobs > 0 && max_blocks > 0) tile_shape(g, num_jobs, max_blocks, out);
+    for (int i = 0; i < 4; ++i) shape[i] = out[i];
+  }
+  return family;
+}
+
 extern "C" int kvmi_kstats_paged(const kvmi_geometry* geom, const kvmi_layer_job* jobs, int32_t num_jobs,
                                  int32_t max_blocks, int32_t* err, kvmi_stream_t stream) {
   using namespace kvmi;
@@ -422,15 +452,13 @@ extern "C" int kvmi_kstats_paged(const kvmi_geometry* geom, const kvmi_layer_job
   if (!jobs || !err) return KVMI_EINVAL;
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   Geo v;
-  if (paired_view(g, &v)) {  // the keys have the same layout in both views: finalize with g
+  const int family = paged_kernels(g, max_blocks, false, &v);
+  if (family == KVMI_KERNELS_MFMA) {  // the keys have the same layout in both views: finalize with g
     rc = mfma_kstats(v, jobs, num_jobs, max_blocks, err, st);
     if (rc) return rc;
-  } else if (mfma_eligible(g)) {
-    rc = mfma_kstats(g, jobs, num_jobs, max_blocks, err, st);
-    if (rc) return rc;
-  } else if (tile_eligible(g, max_blocks)) {
+  } else if (family == KVMI_KERNELS_TILE) {
     return tile_kstats(g, jobs, num_jobs, max_blocks, err, st);  // statistics of both parts + their finalize
-  } else if (!quad_eligible(g)) {
+  } else if (family == KVMI_KERNELS_ROWS) {
     return rows_kstats(g, jobs, num_jobs, max_blocks, err, st);  // statistics of both parts + their finalize
   } else {
     // Statistics need only K: give each workgroup enough blocks that a job has at
@@ -459,10 +487,12 @@ extern "C" int kvmi_encode_paged(const kvmi_geometry* geom, const kvmi_layer_job
   if (!jobs || !err) return KVMI_EINVAL;
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   Geo v;
-  if (paired_view(g, &v)) return mfma_encode(v, jobs, num_jobs, max_blocks, err, st);
-  if (mfma_eligible(g)) return mfma_encode(g, jobs, num_jobs, max_blocks, err, st);
-  if (tile_eligible(g, max_blocks)) return tile_encode(g, jobs, num_jobs, max_blocks, err, st);
-  if (!quad_eligible(g)) return rows_encode(g, jobs, num_jobs, max_blocks, err, st);
+  switch (paged_kernels(g, max_blocks, false, &v)) {
+    case KVMI_KERNELS_MFMA: return mfma_encode(v, jobs, num_jobs, max_blocks, err, st);
+    case KVMI_KERNELS_TILE: return tile_encode(g, jobs, num_jobs, max_blocks, err, st);
+    case KVMI_KERNELS_ROWS: return rows_encode(g, jobs, num_jobs, max_blocks, err, st);
+    default: break;
+  }
   set_valu_bpw(&g);
   dim3 grid((unsigned)((max_blocks + g.bpw - 1) / g.bpw), (unsigned)num_jobs);
   if (g.D == 64) {
@@ -483,10 +513,12 @@ extern "C" int kvmi_decode_paged(const kvmi_geometry* geom, const kvmi_layer_job
   if (!jobs || !err) return KVMI_EINVAL;
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   Geo v;
-  if (paired_view(g, &v)) return mfma_decode(v, jobs, num_jobs, max_blocks, err, st);
-  if (mfma_eligible(g)) return mfma_decode(g, jobs, num_jobs, max_blocks, err, st);
-  if (tile_eligible(g, max_blocks) && tile_decodes(g)) return tile_decode(g, jobs, num_jobs, max_blocks, err, st);
-  if (!quad_eligible(g)) return rows_decode(g, jobs, num_jobs, max_blocks, err, st);
+  switch (paged_kernels(g, max_blocks, true, &v)) {
+    case KVMI_KERNELS_MFMA: return mfma_decode(v, jobs, num_jobs, max_blocks, err, st);
+    case KVMI_KERNELS_TILE: return tile_decode(g, jobs, num_jobs, max_blocks, err, st);
+    case KVMI_KERNELS_ROWS: return rows_decode(g, jobs, num_jobs, max_blocks, err, st);
+    default: break;
+  }
   set_valu_bpw(&g);
   dim3 grid((unsigned)((max_blocks + g.bpw - 1) / g.bpw), (unsigned)num_jobs);
   if (g.D == 64) {

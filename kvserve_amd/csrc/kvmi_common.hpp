@@ -152,13 +152,13 @@ inline int check_geo(const kvmi_geometry* geom, int32_t num_jobs, int32_t max_bl
 //  * MFMA (kvmi_mfma.hip): the transform profile with D in {64, 128}, H dividing 8
 //    (or H = 16 or 32 with a power-of-two S, and 16-byte stream runs) and S*H a
 //    multiple of 32, unless the caller forces the register FWHT (KVMI_F_VALU_FWHT);
-//  * wave tiles (kvmi_tile.hpp; tile_eligible, tile_decodes): the geometries and options
-//    that the first does not take -- D in {64, 80, 96, 112, 128, 160, 192, 224, 256}, up to
-//    32 heads of any count, every quantization axis, no transform -- where a workgroup's
-//    tables and buffers fit 80 KB of LDS.  At 67 MB of raw KV they compress 1.2 - 3.5 times
-//    and decompress 1.1 - 2.5 times as fast as the row kernels, and at 1 MB alike;
+//  * wave tiles (kvmi_tile.hpp; tile_serves): the geometries and options that the first does
+//    not take -- D in {64, 80, 96, 112, 128, 160, 192, 224, 256}, up to 32 heads of any count,
+//    every quantization axis, no transform -- where a workgroup's tables and buffers fit the
+//    LDS (at D = 224, which stages whole rows, up to 3 heads at 4 bits) and a tile is filled
+//    well enough by whole tokens of one block (both sides' times at the rule);
 //  * quad-per-row register FWHT (kvmi_codec.hip): D in {64, 128}, H dividing 128,
-//    H <= 16, when the caller forces it;
+//    H <= 16, when the caller forces it or the tiles of a small block would stay too empty;
 //  * generic rows (kvmi_rows.hip): every other geometry check_geo admits (D even up
 //    to 256 with whole-byte packed rows, split into power-of-two chunks when it is not
 //    one, chunks below 16 channels included; H up to 64), and any geometry when the
@@ -198,8 +198,10 @@ int rows_decode(const Geo& g, const kvmi_layer_job* jobs, int32_t num_jobs, int3
                 hipStream_t st);
 int rows_hadamard(const void* in, void* out, int64_t rows, int32_t H, int32_t D, const uint32_t* signs,
                   int32_t inverse, hipStream_t st);
-bool tile_eligible(const Geo& g, int32_t max_blocks);
-bool tile_decodes(const Geo& g);  // of the eligible ones
+// Whether the wave tiles run the compress (statistics and encode) or the decode of a call that
+// the MFMA kernels do not take, and the launch shape of it (kvmi_paged_kernels).
+bool tile_serves(const Geo& g, int32_t max_blocks, bool decode);
+void tile_shape(const Geo& g, int32_t num_jobs, int32_t max_blocks, int32_t (&out)[4]);
 int tile_kstats(const Geo& g, const kvmi_layer_job* jobs, int32_t num_jobs, int32_t max_blocks, int32_t* err,
                 hipStream_t st);
 int tile_encode(const Geo& g, const kvmi_layer_job* jobs, int32_t num_jobs, int32_t max_blocks, int32_t* err,

@@ -48,7 +48,8 @@ constexpr int kTileMaxH = 32;
 constexpr int kTileWaves = 4;
 constexpr int kTileThreads = 64 * kTileWaves;
 
-// occ: waves per SIMD that the kernel's registers allow
+// Waves per SIMD the registers of the encode and decode kernels are limited to.
+constexpr int tile_occ(int D) { return D <= 128 ? 3 : 2; }
 TileArgs tile_plan(const Geo& g, int32_t max_blocks, int32_t num_jobs, int occ);
 int tile_cus();
 

@@ -60,12 +60,8 @@ __device__ __forceinline__ void unpack8_bits(int bits, const uint8_t* p, float (
   }
 }
 
-// Waves per SIMD the registers are limited to.
-template <int D>
-constexpr int kDecOcc = D <= 128 ? 3 : 2;
-
 template <int D, bool TR, int BITS>
-__global__ __launch_bounds__(kTileThreads, kDecOcc<D>) void tile_decode_kernel(Geo g, TileArgs a,
+__global__ __launch_bounds__(kTileThreads, tile_occ(D)) void tile_decode_kernel(Geo g, TileArgs a,
                                                                                const kvmi_layer_job* __restrict__ jobs,
                                                                                int32_t* __restrict__ err) {
   using TG = TileGeo<D>;
@@ -239,7 +235,7 @@ __global__ __launch_bounds__(kTileThreads, kDecOcc<D>) void tile_decode_kernel(G
 
 template <int D, bool TR, int BITS>
 int launch_b(const Geo& g, const kvmi_layer_job* jobs, int32_t nj, int32_t mb, int32_t* err, hipStream_t st) {
-  const TileArgs a = tile_plan(g, mb, nj, kDecOcc<D>);
+  const TileArgs a = tile_plan(g, mb, nj, tile_occ(D));
   const unsigned gx = (unsigned)(((int64_t)mb * g.S + a.run - 1) / a.run);
   const size_t lds = (size_t)a.off_wave + (size_t)kTileWaves * a.wave_bytes;
   hipLaunchKernelGGL((tile_decode_kernel<D, TR, BITS>), dim3(gx, (unsigned)nj, a.parts == 1 ? 2 : 1), dim3(kTileThreads),

@@ -92,12 +92,8 @@ __device__ __forceinline__ void tile_diff(uint32_t y, float m0, float m1, float&
       : "v"(y), "v"(m0), "v"(m1));
 }
 
-// Waves per SIMD the registers are limited to.
-template <int D>
-constexpr int kEncOcc = D <= 128 ? 3 : 2;
-
 template <int D, bool TR, int BITS>
-__global__ __launch_bounds__(kTileThreads, kEncOcc<D>) void tile_encode_kernel(Geo g, TileArgs a,
+__global__ __launch_bounds__(kTileThreads, tile_occ(D)) void tile_encode_kernel(Geo g, TileArgs a,
                                                                                const kvmi_layer_job* __restrict__ jobs,
                                                                                int32_t* __restrict__ err) {
   using TG = TileGeo<D>;
@@ -284,7 +280,7 @@ __global__ __launch_bounds__(kTileThreads, kEncOcc<D>) void tile_encode_kernel(G
 
 template <int D, bool TR, int BITS>
 int launch_b(const Geo& g, const kvmi_layer_job* jobs, int32_t nj, int32_t mb, int32_t* err, hipStream_t st) {
-  const TileArgs a = tile_plan(g, mb, nj, kEncOcc<D>);
+  const TileArgs a = tile_plan(g, mb, nj, tile_occ(D));
   const unsigned gx = (unsigned)(((int64_t)mb * g.S + a.run - 1) / a.run);
   const size_t lds = (size_t)a.off_wave + (size_t)kTileWaves * a.wave_bytes;
   hipLaunchKernelGGL((tile_encode_kernel<D, TR, BITS>), dim3(gx, (unsigned)nj, a.parts == 1 ? 2 : 1), dim3(kTileThreads),

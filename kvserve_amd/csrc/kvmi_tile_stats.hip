@@ -301,6 +301,9 @@ int tile_cus() {
   return cus;
 }
 
+namespace {
+
+// What the kernels can do: their head sizes, 32-bit offsets, and the LDS of a workgroup.
 bool tile_eligible(const Geo& g, int32_t max_blocks) {
   if (g.flags & (KVMI_F_VALU_FWHT | KVMI_F_ROW_FWHT | kPairedHeads)) return false;
   if (g.H > kTileMaxH) return false;
@@ -316,12 +319,34 @@ bool tile_eligible(const Geo& g, int32_t max_blocks) {
   return lds_bytes(a) <= kMaxLds && slots(g, a) <= max_slots(g);
 }
 
-// Decode of one-token tiles with most rows empty, and of many heads without a transform
-// (whose image runs are short), stays on the row kernels: 960 tokens x 8 layers x 17 heads
-// of 128 channels 45 us against 49, 1024 x 8 x 32 of 64 without transform 26 against 31.
-bool tile_decodes(const Geo& g) {
-  if (kTok / g.H * g.H < 20) return false;
-  return !((g.flags & KVMI_F_NO_TRANSFORM) && g.H > 16);
+// Whether they are the faster ones.  A tile of few rows (small blocks, awkward head counts)
+// costs what a full one does, and what it competes with differs: the quad kernels are about
+// twice as fast as the row kernels, and the row kernels spend next_pow2(D) channels on D.  The
+// rule looks at the geometry alone: with the call's length in it, a request's bytes could
+// depend on the batch it is in.  Compress / decompress (us) of 8 layers x 8192 tokens, the other
+// kernels -> tiles, and the rows of a tile:
+//   quad  8 x 128, S = 1:  8 rows 296 -> 267 / 160 -> 181     S = 2: 16 rows 295 -> 175 / 160 -> 111
+//         4 x 128, S = 2:  8 rows 136 -> 153 /  67 -> 103     S = 4: 16 rows 136 ->  96 /  66 ->  61
+//         1 x 128, S = 8:  8 rows  42 ->  48 /  19 ->  33    S = 16: 16 rows  42 ->  35 /  19 ->  22
+//         8 x 64,  S = 2: 16 rows 131 ->  90 /  51 ->  58; 1024 tokens, 16 x 64, S = 1: 1.18 times the time
+//   rows  5 x 128, S = 1:  5 rows 279 -> 279 / 119 -> 197     S = 2: 10 rows 280 -> 159 / 118 -> 109
+//        10 x 128, S = 1: 10 rows 613 -> 304 / 279 -> 211, but 1024 tokens decompress 1.0 - 1.3 times the time
+//         8 x 96,  S = 1:  8 rows 433 -> 204 / 168 -> 137    12 x 96, S = 1: 12 rows 759 -> 264 / 296 -> 190
+// Short calls (up to a few hundred tokens) of few heads of 160 channels and more take 1 - 5 us
+// longer than on the other kernels however full the tiles are: the latency of one tile.
+bool tile_faster(const Geo& g, bool decode) {
+  const int rows = shape(g, 1).T * g.H;
+  if (decode && (g.flags & KVMI_F_NO_TRANSFORM) && g.H > 16) return false;  // short image runs: 1024 x 8 x 32 of 64 26 -> 31 us
+  if (quad_eligible(g)) return decode ? rows >= 20 : rows * g.D >= 16 * 128;
+  const bool pow2 = next_pow2(g.D) == g.D;
+  if (decode) return rows >= 20 || (!pow2 && g.H <= 16 && rows >= 12);  // 17 heads of 128, 960 x 8: 45 -> 49 us
+  return rows >= (pow2 ? 10 : 8);
+}
+
+}  // namespace
+
+bool tile_serves(const Geo& g, int32_t max_blocks, bool decode) {
+  return tile_eligible(g, max_blocks) && tile_faster(g, decode);
 }
 
 TileArgs tile_plan(const Geo& g, int32_t max_blocks, int32_t num_jobs, int occ) {
@@ -350,6 +375,11 @@ TileArgs tile_plan(const Geo& g, int32_t max_blocks, int32_t num_jobs, int occ) 
   // few tiles: K and V in workgroups of their own, half the serial work of a wave
   a.parts = (tokens + a.run - 1) / a.run * num_jobs * 2 <= resident(a) ? 1 : 2;
   return a;
+}
+
+void tile_shape(const Geo& g, int32_t num_jobs, int32_t max_blocks, int32_t (&out)[4]) {
+  const TileArgs a = tile_plan(g, max_blocks, num_jobs, tile_occ(g.D));
+  out[0] = a.T, out[1] = a.ST / a.T, out[2] = a.run, out[3] = a.parts;
 }
 
 int tile_kstats(const Geo& g, const kvmi_layer_job* jobs, int32_t num_jobs, int32_t max_blocks, int32_t*,
