@@ -526,7 +526,13 @@ unsigned v3_grid(int64_t rows, int H) {
 
 // Workgroups of a part of the quantizing pass: beyond what the chip holds at once (4 a CU,
 // both parts together) each takes two passes, the second one's rows in flight during the first.
-unsigned v3_qgrid(unsigned passes) { return passes > 512 ? (passes + 1) / 2 : passes; }
+// K's passes are by head, so that a few rows of many heads make more of them than V's (one row
+// of 64 heads of 128: 64 passes in one workgroup 183 us, in 64 of them 22).
+unsigned v3_qgrid(int64_t rows, int H) {
+  const int64_t kpasses = (rows + kV3Rows - 1) / kV3Rows * H;
+  const unsigned v = v3_grid(rows, H), passes = kpasses > (int64_t)v ? (unsigned)kpasses : v;
+  return passes > 512 ? (passes + 1) / 2 : passes;
+}
 
 // Workgroups of the K statistics pass, i.e. the K partials one call writes and reads.
 unsigned v3_kgrid(int64_t rows, int H) {
@@ -540,8 +546,7 @@ int v3_compress_launch(const void* x, int64_t rows, int32_t H, int32_t D, const 
                        const float* levels, const int32_t* vgroup, uint8_t* q, const V3Meta& meta, uint32_t* kpart,
                        hipStream_t st) {
   V3Shape sh{rows, H, (float)(1.0 / __builtin_sqrt((double)D))};
-  const unsigned g = v3_grid(rows, H);
-  const unsigned gk = v3_kgrid(rows, H), gq = v3_qgrid(g);
+  const unsigned gk = v3_kgrid(rows, H), gq = v3_qgrid(rows, H);
   const size_t klds = (size_t)2 * H * D * 4;
   const uint16_t* xs = static_cast<const uint16_t*>(x);
   const unsigned gf = (unsigned)((H * D + 3) / 4);  // 4 channels per workgroup

@@ -84,3 +84,31 @@ def test_scales_without_a_finite_value_give_zero(cuda):
     q, _, _ = _compress(cuda, t.to(cuda), lv, torch.tensor([0, 1], dtype=torch.int32, device=cuda), D, False)
     assert not q[1, 3, 0].any() and not q[1, 5, 1].any() and q[1, 3, 1].any() and q[1, 4].any()
     assert not q[0, :, 0].any()  # one infinity spreads over every channel of its head's row
+
+
+@pytest.mark.parametrize("H,D", [(64, 128), (32, 64)])
+def test_a_few_rows_of_many_heads_take_no_longer_than_a_pass_of_them(cuda, H, D):
+    """K's passes are by head: one row of H heads is H passes, which run side by side.  The least
+    of 20 timings of one row is within 1.5 times that of 64 rows, which have the same passes with
+    every lane in use (one workgroup running them in turn took 5 to 8 times as long)."""
+    lv, group = torch.full((2, H), 12.0, device=cuda), torch.zeros(H, dtype=torch.int32, device=cuda)
+    lib, least = _lib.load(), {}
+    for rows in (1, 64):
+        x = torch.randn((2, rows, H, D), generator=torch.Generator().manual_seed(1)).to(torch.bfloat16).to(cuda)
+        signs = torch.zeros((H, D // 32), dtype=torch.int32, device=cuda)
+        q, k = torch.empty_like(x, dtype=torch.uint8), torch.empty((2, H, D), device=cuda)
+        v = torch.empty((2, rows, H), device=cuda)
+        ws = torch.empty(int(lib.kvmi_v3_scratch_bytes(rows, H, D)), dtype=torch.uint8, device=cuda)
+        stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+        times = []
+        for _ in range(20):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            for _ in range(10):
+                _lib.check(lib.kvmi_v3_compress(x.data_ptr(), rows, H, D, signs.data_ptr(), lv.data_ptr(), group.data_ptr(),
+                                                q.data_ptr(), k.data_ptr(), v.data_ptr(), ws.data_ptr(), stream), "compress")
+            b.record()
+            b.synchronize()
+            times.append(a.elapsed_time(b))
+        least[rows] = min(times)
+    assert least[1] <= 1.5 * least[64], least
