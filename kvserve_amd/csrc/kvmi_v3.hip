@@ -524,14 +524,18 @@ unsigned v3_grid(int64_t rows, int H) {
   return (unsigned)(passes > 0 ? passes : 1);
 }
 
-// Workgroups of a part of the quantizing pass: beyond what the chip holds at once (4 a CU,
-// both parts together) each takes two passes, the second one's rows in flight during the first.
-// K's passes are by head, so that a few rows of many heads make more of them than V's (one row
-// of 64 heads of 128: 64 passes in one workgroup 183 us, in 64 of them 22).
-unsigned v3_qgrid(int64_t rows, int H) {
+// Workgroups of a part of the quantizing pass.  K's passes are by head, so that a few rows of
+// many heads make more of them than V's (one row of 64 heads of 128: 64 passes in one workgroup
+// 183 us, in 64 of them 22).  At D = 128 at most what the chip holds at once (4 workgroups a CU,
+// both parts together), each walking its passes with the next one's rows in flight: 4 x the
+// passes, 32768 rows of 8 heads, compress 94 us, two passes each 111, one 111.  At D = 64, whose
+// workgroups are lighter, one pass each up to 2048, then two (16384 rows of 32 heads: 109 us, one
+// 112, 512 workgroups 116; 4096 of 16: 23.2, two 24.0).
+unsigned v3_qgrid(int64_t rows, int H, int D) {
   const int64_t kpasses = (rows + kV3Rows - 1) / kV3Rows * H;
   const unsigned v = v3_grid(rows, H), passes = kpasses > (int64_t)v ? (unsigned)kpasses : v;
-  return passes > 512 ? (passes + 1) / 2 : passes;
+  if (D == 128) return passes > 512 ? 512 : passes;
+  return passes > 2048 ? (passes + 1) / 2 : passes;
 }
 
 // Workgroups of the K statistics pass, i.e. the K partials one call writes and reads.
@@ -546,7 +550,7 @@ int v3_compress_launch(const void* x, int64_t rows, int32_t H, int32_t D, const 
                        const float* levels, const int32_t* vgroup, uint8_t* q, const V3Meta& meta, uint32_t* kpart,
                        hipStream_t st) {
   V3Shape sh{rows, H, (float)(1.0 / __builtin_sqrt((double)D))};
-  const unsigned gk = v3_kgrid(rows, H), gq = v3_qgrid(rows, H);
+  const unsigned gk = v3_kgrid(rows, H), gq = v3_qgrid(rows, H, D);
   const size_t klds = (size_t)2 * H * D * 4;
   const uint16_t* xs = static_cast<const uint16_t*>(x);
   const unsigned gf = (unsigned)((H * D + 3) / 4);  // 4 channels per workgroup

@@ -62,9 +62,10 @@ def test_symbols_on_the_boundaries(cuda, D, exponent, levels):
     assert torch.equal(q16, q) and torch.equal(k16, k.half()) and torch.equal(v16, v.half())
 
 
-@pytest.mark.parametrize("rows,H,D", [(4111, 8, 128), (16391, 2, 64), (2049, 16, 128)])
-def test_layers_of_two_passes_a_workgroup(cuda, rows, H, D):
-    """More passes than the chip holds at once, an odd number of them, the last one ragged."""
+@pytest.mark.parametrize("rows,H,D", [(4111, 8, 128), (16391, 2, 64), (2049, 16, 128), (9031, 8, 128), (16403, 8, 64)])
+def test_layers_of_several_passes_a_workgroup(cuda, rows, H, D):
+    """More passes than workgroups (two or three each), or an odd number of them, the last one
+    ragged."""
     t = torch.randn((2, rows, H, D), generator=torch.Generator().manual_seed(rows)).to(torch.bfloat16)
     kl, vl = [16.0] * H, [12.0, 6.0] * (H // 2)
     ref_q, ref_m = fv.compress_layer(t.view(torch.int16).numpy().view(np.uint16), kp.rademacher_signs(SEED, 1, H, D), kl, vl)
