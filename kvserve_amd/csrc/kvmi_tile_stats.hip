@@ -268,8 +268,8 @@ int slots(const Geo& g, const TileArgs& a) {
   return a.runs * ((a.ST * RB * (a.runs == 1 && (g.flags & KVMI_F_NATIVE_LAYOUT) ? g.H : 1) + 15) / 16);
 }
 
-constexpr int kMaxLds = 80 * 1024;  // two workgroups a CU
-constexpr int kStaticLds = 1024;       // TileTables and the like, rounded up
+constexpr int kStaticLds = 1024;                  // TileTables and the like, rounded up
+constexpr int kMaxLds = 80 * 1024 - kStaticLds;   // two workgroups a CU
 // A wave's image grows, tile by tile, until a head's run in the stream is kRunBytes long (or
 // the image kImageBytes, or a wave would be left without a super-tile).  Longer runs beat
 // more resident workgroups: 16 layers x 4096 tokens x 8 heads of 128 channels, 4 bits, K per
@@ -304,7 +304,9 @@ int tile_cus() {
 namespace {
 
 // What the kernels can do: their head sizes, 32-bit offsets, and the LDS of a workgroup.
-bool tile_eligible(const Geo& g, int32_t max_blocks) {
+// Decode needs two workgroups a CU (8 layers x 1024 tokens of 10 heads of 256, both parts by
+// channel: one 73 us, the row kernels 48); compress still gains with one (4096 tokens 568 -> 413).
+bool tile_eligible(const Geo& g, int32_t max_blocks, bool decode) {
   if (g.flags & (KVMI_F_VALU_FWHT | KVMI_F_ROW_FWHT | kPairedHeads)) return false;
   if (g.H > kTileMaxH) return false;
   switch (g.D) {
@@ -316,7 +318,7 @@ bool tile_eligible(const Geo& g, int32_t max_blocks) {
   if (tokens * g.H * g.D * g.bits / 8 >= (1ll << 32)) return false;        // 32-bit offsets in a part's stream
   if ((g.flags & KVMI_F_NO_TRANSFORM) && g.H * g.D / 8 > kTileThreads) return false;
   const TileArgs a = shape(g, 1);
-  return lds_bytes(a) <= kMaxLds && slots(g, a) <= max_slots(g);
+  return lds_bytes(a) <= kMaxLds + (decode ? 0 : kStaticLds) && slots(g, a) <= max_slots(g);
 }
 
 // Whether they are the faster ones.  A tile of few rows (small blocks, awkward head counts)
@@ -346,7 +348,7 @@ bool tile_faster(const Geo& g, bool decode) {
 }  // namespace
 
 bool tile_serves(const Geo& g, int32_t max_blocks, bool decode) {
-  return tile_eligible(g, max_blocks) && tile_faster(g, decode);
+  return tile_eligible(g, max_blocks, decode) && tile_faster(g, decode);
 }
 
 TileArgs tile_plan(const Geo& g, int32_t max_blocks, int32_t num_jobs, int occ) {

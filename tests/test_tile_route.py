@@ -37,6 +37,8 @@ def kernels(H, D, S, bits=4, flags=0, blocks=64, jobs=8):
     (6, 96, 1, 0, R, R), (8, 96, 1, 0, T, R), (12, 96, 1, 0, T, T), (6, 96, 2, 0, T, T), (6, 96, 16, 0, T, T), (1, 96, 4, 0, R, R),
     # one token a tile; many heads without a transform decode on the row kernels
     (17, 96, 16, 0, T, R), (20, 96, 16, 0, T, T), (32, 64, 1, KTOK, T, T), (32, 64, 16, PLAIN, T, R), (33, 64, 16, 0, R, R),
+    # the LDS of a workgroup: at most one a CU compresses, two decode
+    (10, 256, 16, KTOK | VCH, T, T), (10, 256, 16, VCH, T, R), (12, 256, 16, VCH, R, R), (3, 224, 16, 0, T, T), (4, 224, 16, 0, R, R),
     # forced families
     (6, 96, 16, _lib.F_ROW_FWHT, R, R), (8, 128, 16, _lib.F_VALU_FWHT, Q, Q),
 ])
