@@ -125,6 +125,7 @@ __global__ __launch_bounds__(kTileThreads, tile_occ(D)) void tile_encode_kernel(
   if (TR) tile_signs<D>(smask, job.signs, H);
   __syncthreads();
   tile_positions(T, H);
+  tile_groups(T, H, a.tabs);
   const int tab1 = (a.tabs & 1) ? H * (D + 4) : 0;  // V's table behind K's
   if ((a.tabs & 1) && part0 == 0) tile_consts<D, true>(kc, T, g, job.kmeta, 0);
   if ((a.tabs & 2) && part1 == 2) tile_consts<D, true>(kc + tab1, T, g, job.vmeta, 1);
