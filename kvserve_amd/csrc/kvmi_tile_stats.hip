@@ -1,5 +1,7 @@
 // Statistics pass of the wave-tile kernels (kvmi_tile.hpp) for the parts on the channel or
 // tensor axis, and the launch shape of all three passes.
+#include <algorithm>
+
 #include "kvmi_tile.hpp"
 
 namespace kvmi {
@@ -10,8 +12,9 @@ constexpr int kStatTok = 32;  // tokens of a statistics tile
 // A tile is 32 consecutive tokens of one head (rows 2 H D bytes apart; past the run its last
 // token again, which min and max ignore), transformed in orientation N: a lane holds 16
 // rows of one channel, so a head's running minimum and maximum are one pair per output tile.
-// The workgroup's (head, tile) pairs are split evenly over its waves, head by head; where a
-// wave leaves a head it adds the pairs to the workgroup's LDS keys.  Bound by its reads and
+// The (head, tile) pairs of a run are split evenly over the waves of its workgroups (several in
+// short calls, blockIdx.z), head by head; where a wave leaves a head it adds the pairs to the
+// workgroup's LDS keys.  Bound by its reads and
 // their latency (8 waves a CU): K of 16 layers x 4080 tokens x 6 heads of 96 channels (75 MB)
 // 47 us on the row kernels, 20 here (3.8 TB/s); V of 16 x 4096 x 8 of 128 (134 MB) 72 -> 30 us.
 template <int D>
@@ -24,7 +27,7 @@ __global__ __launch_bounds__(kTileThreads, D <= 80 ? 4 : D <= 128 ? 3 : 2) void 
   const int ntok = job.num_blocks * S, tok0 = blockIdx.x * a.run;
   if (tok0 >= ntok) return;
   const int tok_end = min(ntok, tok0 + a.run);
-  const int part = (a.tabs == 3) ? (int)blockIdx.z : (a.tabs >> 1);
+  const int parts = a.tabs == 3 ? 2 : 1, part = parts == 2 ? (int)blockIdx.z & 1 : (a.tabs >> 1);
   const bool channel = part_axis(g.flags, part) == kAxChannel;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int l = threadIdx.x & 63, hl = l >> 5, r = l & 31;
@@ -63,7 +66,8 @@ __global__ __launch_bounds__(kTileThreads, D <= 80 ? 4 : D <= 128 ? 3 : 2) void 
   }
   const uint16_t* pool = reinterpret_cast<const uint16_t*>(job.pool) + (part ? job.pool_part_stride : 0);
   const int nk = (tok_end - tok0 + kStatTok - 1) / kStatTok, items = nk * H;
-  const int first = wave * items / kTileWaves, end = (wave + 1) * items / kTileWaves;
+  const int waves = kTileWaves * (int)gridDim.z / parts, w = kTileWaves * ((int)blockIdx.z / parts) + wave;
+  const int first = w * items / waves, end = (w + 1) * items / waves;
   // Row r's token index in the pool goes through LDS to the lanes that load the row; the
   // block ids of a tile are loaded one tile earlier than its rows.
   int* ptok = reinterpret_cast<int*>(tb + TG::kBuf);
@@ -400,7 +404,12 @@ int tile_kstats(const Geo& g, const kvmi_layer_job* jobs, int32_t num_jobs, int3
                                               : 2 * kPlainAhead * (kTileThreads / (g.H * g.D / 8));
   run = run < least ? least : (run + unit - 1) / unit * unit;
   a.run = (int)(run > tokens ? (tokens + unit - 1) / unit * unit : run);
-  const dim3 grid((unsigned)((tokens + a.run - 1) / a.run), (unsigned)num_jobs, parts);
+  // a short call leaves the chip idle and a wave walks several heads: more workgroups a run, down
+  // to a tile a wave (8 layers x 64 tokens x 10 heads of 256: 29 -> 16 us, row kernels 16)
+  const int64_t groups = (tokens + a.run - 1) / a.run * num_jobs * parts, items = (int64_t)(a.run / kStatTok) * g.H;
+  int64_t share = 1;
+  if (tr) share = std::max<int64_t>(1, std::min(want / groups, (items + kTileWaves - 1) / kTileWaves));
+  const dim3 grid((unsigned)((tokens + a.run - 1) / a.run), (unsigned)num_jobs, (unsigned)(parts * share));
   const size_t keys = (size_t)2 * g.H * g.D * 4;
   int rc;
   if (tr) {
