@@ -337,16 +337,20 @@ bool tile_eligible(const Geo& g, int32_t max_blocks, bool decode) {
 //         8 x 64,  S = 2: 16 rows 131 ->  90 /  51 ->  58; 1024 tokens, 16 x 64, S = 1: 1.18 times the time
 //   rows  5 x 128, S = 1:  5 rows 279 -> 279 / 119 -> 197     S = 2: 10 rows 280 -> 159 / 118 -> 109
 //        10 x 128, S = 1: 10 rows 613 -> 304 / 279 -> 211, but 1024 tokens decompress 1.0 - 1.3 times the time
-//         8 x 96,  S = 1:  8 rows 433 -> 204 / 168 -> 137    12 x 96, S = 1: 12 rows 759 -> 264 / 296 -> 190
-// Short calls (up to a few hundred tokens) of few heads of 160 channels and more take 1 - 5 us
-// longer than on the other kernels however full the tiles are: the latency of one tile.
+//         8 x 96,  S = 1:  8 rows 433 -> 204 / 168 -> 137    12 x 96, S = 1: 12 rows 759 -> 254 / 296 -> 190
+// Short calls of few large heads stay slower than on the other kernels, however full the tiles
+// are: the latency of one tile.  Up to about 1000 tokens of 1 - 5 heads decompress takes 1 - 3 us
+// longer from 160 channels on (1 x 224 at 528 x 4: 7.9 -> 12.4), compress 3 - 8 us at 256 (5 heads
+// at 128 x 8: 22 -> 30).
 bool tile_faster(const Geo& g, bool decode) {
   const int rows = shape(g, 1).T * g.H;
   if (decode && (g.flags & KVMI_F_NO_TRANSFORM) && g.H > 16) return false;  // short image runs: 1024 x 8 x 32 of 64 26 -> 31 us
   if (quad_eligible(g)) return decode ? rows >= 20 : rows * g.D >= 16 * 128;
-  const bool pow2 = next_pow2(g.D) == g.D;
-  if (decode) return rows >= 20 || (!pow2 && g.H <= 16 && rows >= 12);  // 17 heads of 128, 960 x 8: 45 -> 49 us
-  return rows >= (pow2 ? 10 : 8);
+  const bool waste = 4 * next_pow2(g.D) >= 5 * g.D;  // of the row kernels: 80, 96, 160 and 192 channels
+  // 12 rows: only at 4 bits, which has code of its own (1770 x 8 of 12 x 96 at 5 bits 50 -> 74 us), and
+  // not with one token a tile beyond 16 heads (960 x 8 of 17 x 128 45 -> 49)
+  if (decode) return rows >= 20 || (waste && g.bits == 4 && g.H <= 16 && rows >= 12);
+  return rows >= (waste ? 8 : 10);
 }
 
 }  // namespace

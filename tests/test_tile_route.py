@@ -35,6 +35,7 @@ def kernels(H, D, S, bits=4, flags=0, blocks=64, jobs=8):
     (1, 128, 1, KTOK, R, R), (8, 128, 1, KTOK | VCH, R, R), (8, 128, 2, KTOK | VCH, T, R), (8, 128, 4, KTOK, T, T),
     (5, 128, 1, 0, R, R), (5, 128, 2, 0, T, R), (10, 128, 1, 0, T, R), (12, 128, 2, 0, T, T),
     (6, 96, 1, 0, R, R), (8, 96, 1, 0, T, R), (12, 96, 1, 0, T, T), (6, 96, 2, 0, T, T), (6, 96, 16, 0, T, T), (1, 96, 4, 0, R, R),
+    (12, 112, 1, 0, T, R), (8, 112, 1, 0, R, R), (1, 192, 16, 0, T, T), (1, 224, 16, 0, T, R),
     # one token a tile; many heads without a transform decode on the row kernels
     (17, 96, 16, 0, T, R), (20, 96, 16, 0, T, T), (32, 64, 1, KTOK, T, T), (32, 64, 16, PLAIN, T, R), (33, 64, 16, 0, R, R),
     # the LDS of a workgroup: at most one a CU compresses, two decode
@@ -59,3 +60,9 @@ def test_bad_geometry_is_refused():
     geo = _lib.Geometry(block_size=16, num_heads=65, head_dim=128, bits=4, max_groups=1)
     assert _lib.load().kvmi_paged_kernels(ctypes.byref(geo), 1, 1, 0, None) == _lib.EINVAL
     assert _lib.load().kvmi_paged_kernels(None, 1, 1, 0, None) == _lib.EINVAL
+
+
+def test_widths_other_than_4_bits_decode_on_tiles_from_20_rows():
+    for bits, decode in ((4, T), (5, R), (3, R)):
+        assert [f for f, _ in kernels(12, 96, 1, bits=bits)] == [T, decode]
+        assert [f for f, _ in kernels(6, 96, 16, bits=bits)] == [T, T]
