@@ -3,8 +3,9 @@ axis_key / axis_value, kvserve_quantizer.py:136-139): every (axis_key, axis_valu
 through the C-ABI paged kernels against the oracle, and the KVServeQuantizer operator
 against the golden vectors the reference itself wrote (tests/golden/quantizer_axes.npz).
 
-Non-default axes run on the generic row kernels, whose FWHT stage order is the oracle's:
-symbols, metadata and the decompressed KV are bit-exact."""
+The generic row kernels (fwht="rows") run the oracle's FWHT stage order: symbols, metadata and
+the decompressed KV are bit-exact.  The default kernels (wave tiles for the non-default axes)
+add in another fp32 order and are held to the configuration bars of test_gpu_configs.py."""
 
 from pathlib import Path
 
@@ -13,6 +14,7 @@ import pytest
 import torch
 
 from oracle import kvpipe as kp
+from test_gpu_configs import _check_layer
 
 pytestmark = pytest.mark.gpu
 
@@ -32,6 +34,16 @@ def _oracle_profile(p):
 @pytest.mark.parametrize("axes", PAIRS, ids=["-".join(p) for p in PAIRS])
 @pytest.mark.parametrize("H,D,bits,layout", [(8, 128, 4, "permuted"), (6, 96, 5, "native")])
 def test_axes_match_oracle_exactly(cuda, axes, H, D, bits, layout):
+    _axes_vs_oracle(cuda, axes, H, D, bits, layout, "rows")
+
+
+@pytest.mark.parametrize("axes", PAIRS, ids=["-".join(p) for p in PAIRS])
+@pytest.mark.parametrize("H,D,bits,layout", [(8, 128, 4, "permuted"), (6, 96, 5, "native")])
+def test_axes_on_the_default_kernels(cuda, axes, H, D, bits, layout):
+    _axes_vs_oracle(cuda, axes, H, D, bits, layout, "mfma")
+
+
+def _axes_vs_oracle(cuda, axes, H, D, bits, layout, fwht):
     from kvserve_amd.engine import FusedKVCodec, check_packet
     from kvserve_amd.profiles import section_profile, whole_layer_profile
     from kvserve_amd.workloads import kv_blocks
@@ -46,10 +58,10 @@ def test_axes_match_oracle_exactly(cuda, axes, H, D, bits, layout):
     prof = [section_profile([bool(v) for v in torch.randint(0, 2, (H,), generator=g)], top, top - 1,
                             max(2, top - 3), max(2, top - 4)) for _ in range(L - 1)]
     prof.append(whole_layer_profile(H, max(2, top - 2), top, is_low=True))  # one section
-    print(f"axes {axes} H={H} D={D} bits={bits} {layout}", flush=True)
+    print(f"axes {axes} H={H} D={D} bits={bits} {layout} {fwht}", flush=True)
     pools = [p.to(cuda) for p in pools]
     dev_ids = ids.to(torch.int32).to(cuda)
-    codec = FusedKVCodec(H, D, S, bits, 0xC0FEBABE, layout=layout, axes=axes)
+    codec = FusedKVCodec(H, D, S, bits, 0xC0FEBABE, layout=layout, axes=axes, fwht=fwht)
     packet = codec.compress(pools, dev_ids, prof)
     check_packet(packet)
     dst = [torch.zeros_like(p) for p in pools]
@@ -59,6 +71,9 @@ def test_axes_match_oracle_exactly(cuda, axes, H, D, bits, layout):
     stream = packet.streams[0].cpu().numpy()
     for l in range(L):
         x = _bits(pools[l][:, dev_ids.long()])
+        if fwht == "mfma":
+            _check_layer(packet, l, x, _bits(dst[l][:, dev_ids.long()]))
+            continue
         op = _oracle_profile(packet.profiles[l])
         ch = kp.compress_request([x], list(range(B)), [op], packet.seed, bits, layout=layout,
                                  layer_ids=[packet.layer_ids[l]], chunks=[(0, 1)], axes=axes)[0]

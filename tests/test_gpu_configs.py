@@ -77,31 +77,28 @@ def _check_layer(packet, l: int, x_bits: np.ndarray, out_bits=None):
     B = x_bits.shape[1]
     prof = _oracle_profile(packet.profiles[l])
     lid = packet.layer_ids[l]
-    ch = kp.compress_request([x_bits], list(range(B)), [prof], packet.seed, packet.bits, layout=packet.layout,
-                             layer_ids=[lid], chunks=[(0, 1)])[0]
+    how = dict(layout=packet.layout, layer_ids=[lid], axes=packet.axes)
+    ch = kp.compress_request([x_bits], list(range(B)), [prof], packet.seed, packet.bits, chunks=[(0, 1)], **how)[0]
     d = np.abs(_layer_symbols(packet, l).astype(np.int16) - ch.symbols.reshape(-1).astype(np.int16))
     assert d.max() <= 1 and np.count_nonzero(d) <= SYM_MISMATCH_FRAC * d.size, (l, d.max(), np.count_nonzero(d))
     m = ch.metas[0]
-    km = packet.kmeta[l].float().cpu().numpy()
-    assert np.array_equal(km[0], m.kmin) and np.array_equal(km[1], m.kscale), l
-    G = m.vmin.shape[0]
-    vm = packet.vmeta[l].float().cpu().numpy()
-    assert np.array_equal(vm[0, :G], m.vmin) and np.array_equal(vm[1, :G], m.vscale), l
+    own_meta = []
+    for t, mn, sc in ((packet.kmeta[l], m.kmin, m.kscale), (packet.vmeta[l], m.vmin, m.vscale)):
+        got = t.float().cpu().numpy()[:, :mn.shape[0]]
+        assert np.array_equal(got[0], mn) and np.array_equal(got[1], sc), l
+        own_meta += [got[0], got[1]]
     if out_bits is not None:
         ref = np.zeros_like(x_bits)
-        kp.decompress_request([ch], [ref], list(range(B)), [prof], packet.seed, packet.bits, layout=packet.layout,
-                              layer_ids=[lid])
+        kp.decompress_request([ch], [ref], list(range(B)), [prof], packet.seed, packet.bits, **how)
         x, xr = kp.bf16_to_f32(out_bits), kp.bf16_to_f32(ref)
         for part in range(2):
             rel = np.abs(x[part] - xr[part]).max() / np.abs(xr[part]).max()
             assert rel <= DEQ_REL_TOL, (l, part, rel)
         # the GPU's own stream and metadata decoded by the oracle: the same symbols and
         # constants, so only the fp32 summation order of the inverse transform differs
-        own = kp.Chunk(0, 1, np.empty(ch.symbols.shape, np.uint8), _layer_stream(packet, l),
-                       [kp.LayerMeta(km[0], km[1], vm[0, :G], vm[1, :G])])
+        own = kp.Chunk(0, 1, np.empty(ch.symbols.shape, np.uint8), _layer_stream(packet, l), [kp.LayerMeta(*own_meta)])
         mine = np.zeros_like(x_bits)
-        kp.decompress_request([own], [mine], list(range(B)), [prof], packet.seed, packet.bits, layout=packet.layout,
-                              layer_ids=[lid])
+        kp.decompress_request([own], [mine], list(range(B)), [prof], packet.seed, packet.bits, **how)
         _assert_within_one_ulp(out_bits, mine, OWN_DECODE_ULP_FRAC, l)
 
 
@@ -359,7 +356,7 @@ def test_config5_full_size_batch_sampled_matches_oracle(cuda, path):
     (16, 16, 128, 4),  # 16 heads: wide-head MFMA kernels (2 tokens per tile)
     (32, 16, 128, 4),  # 32 heads: one token per tile, head-major statistics tiles
     (32, 16, 64, 2),
-    (32, 16, 64, 3),   # 24-byte stream runs at 32 heads: the generic row kernels
+    (32, 16, 64, 3),   # 24-byte stream runs at 32 heads: not the MFMA kernels
     (16, 32, 64, 3),
     (32, 1, 128, 4),   # one-token blocks: a statistics tile spans 32 blocks
     (8, 16, 64, 5),
@@ -403,7 +400,7 @@ def _geometry_vs_oracle(cuda, H, S, D, bits, layout="permuted"):
         _check_layer(packet, l, x[l], _bits(dst[l][:, ids.to(cuda).long()]))
 
 
-@pytest.mark.parametrize("H,S,D,bits,layout", [
+GENERIC = [
     (32, 16, 128, 4, "permuted"),  # 32 KV heads (MHA model, one rank)
     (6, 16, 128, 4, "permuted"),   # H not dividing 128
     (8, 16, 256, 4, "permuted"),   # D = 256
@@ -419,13 +416,23 @@ def _geometry_vs_oracle(cuda, H, S, D, bits, layout="permuted"):
     (5, 32, 70, 4, "native"),      # D = 64 + 4 + 2
     (2, 16, 6, 4, "permuted"),     # D = 4 + 2: the whole row in one partial lane
     (6, 16, 100, 6, "permuted"),
-])
+]
+
+
+@pytest.mark.parametrize("H,S,D,bits,layout", GENERIC)
 def test_generic_geometries_match_oracle_exactly(cuda, H, S, D, bits, layout):
     """The generic row kernels (kvmi_rows.hip) run the oracle's FWHT stage order, so
-    symbols, metadata and the decompressed KV are bit-exact with the oracle.  (32 heads
-    at D = 128 and D = 256 would take the MFMA kernels: the row kernels are forced.)"""
-    _rows_exact(cuda, H, S, D, bits, layout,
-                fwht="rows" if (H in (16, 32) and D in (64, 128)) or (D == 256 and H <= 16) else None)
+    symbols, metadata and the decompressed KV are bit-exact with the oracle."""
+    _rows_exact(cuda, H, S, D, bits, layout, fwht="rows")
+
+
+@pytest.mark.parametrize("H,S,D,bits,layout", GENERIC)
+def test_generic_geometries_match_oracle(cuda, H, S, D, bits, layout):
+    """The kernels these geometries run by themselves (wave tiles where kvmi_paged_kernels
+    says so, which add in another fp32 order), within the configuration bars."""
+    packet, pools, dst, dev_ids = _generic_round_trip(cuda, H, S, D, bits, layout, None)
+    for l in range(len(pools)):
+        _check_layer(packet, l, _bits(pools[l][:, dev_ids.long()]), _bits(dst[l][:, dev_ids.long()]))
 
 
 @pytest.mark.parametrize("H,S,D,bits", [(8, 16, 128, 4), (8, 16, 64, 4), (4, 32, 128, 3)])
@@ -435,7 +442,7 @@ def test_forced_row_kernels_match_oracle_exactly(cuda, H, S, D, bits):
     _rows_exact(cuda, H, S, D, bits, "permuted", fwht="rows")
 
 
-def _rows_exact(cuda, H, S, D, bits, layout, fwht=None):
+def _generic_round_trip(cuda, H, S, D, bits, layout, fwht):
     from kvserve_amd.engine import FusedKVCodec, check_packet
     from kvserve_amd.profiles import section_profile
     from kvserve_amd.workloads import kv_blocks
@@ -458,7 +465,13 @@ def _rows_exact(cuda, H, S, D, bits, layout, fwht=None):
     dst = [torch.zeros_like(p) for p in pools]
     codec.decompress(packet, dst, dev_ids)
     torch.cuda.synchronize()
-    for l in range(L):
+    return packet, pools, dst, dev_ids
+
+
+def _rows_exact(cuda, H, S, D, bits, layout, fwht):
+    packet, pools, dst, dev_ids = _generic_round_trip(cuda, H, S, D, bits, layout, fwht)
+    B = dev_ids.numel()
+    for l in range(len(pools)):
         x = _bits(pools[l][:, dev_ids.long()])
         oprof = _oracle_profile(packet.profiles[l])
         ch = kp.compress_request([x], list(range(B)), [oprof], packet.seed, bits, layout=layout,

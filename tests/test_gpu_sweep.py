@@ -89,7 +89,7 @@ def test_sweep_matches_oracle(cuda, H, S, D, bits, L, B, layout, path, fwht, see
 
 
 def test_symbol_at_the_top_of_the_width_is_rejected_like_the_reference(cuda):
-    """128 levels at 7 bits, D = 96 (the generic row kernels, bit-exact with the oracle):
+    """128 levels at 7 bits, D = 96 on the row kernels, which are bit-exact with the oracle:
     on this seeded request the oracle rounds some element to symbol 128 and rejects the
     layer; the engine's error check after the run raises the reference's bitpack error.
     With 127 levels the same request compresses and matches the oracle."""
@@ -109,7 +109,7 @@ def test_symbol_at_the_top_of_the_width_is_rejected_like_the_reference(cuda):
     for levels, rejects in ((128, True), (127, False)):
         prof = [per_head_profile([levels] * H, [levels] * H)]
         print(f"top of width: H={H} D={D} bits={bits} levels={levels}", flush=True)
-        codec = FusedKVCodec(H, D, S, bits, 0xC0FEBABE, layout="native")
+        codec = FusedKVCodec(H, D, S, bits, 0xC0FEBABE, layout="native", fwht="rows")
         if rejects:
             with pytest.raises(ValueError, match="symbol exceeds bitpack_bits"):
                 kp.compress_request([x], list(range(B)), [_oracle_profile(prof[0])], codec.seed, bits,
@@ -141,13 +141,24 @@ def _axes_cases(n: int, seed: int):
     return out
 
 
-@pytest.mark.parametrize("H,S,D,bits,ak,av,L,B,layout,seed",
-                         _axes_cases(int(os.environ.get("KVSERVE_AMD_SWEEP_CASES", "48")) // 2, 20261203))
+AXES_SWEEP = _axes_cases(int(os.environ.get("KVSERVE_AMD_SWEEP_CASES", "48")) // 2, 20261203)
+
+
+@pytest.mark.parametrize("H,S,D,bits,ak,av,L,B,layout,seed", AXES_SWEEP)
 def test_axes_sweep_matches_oracle_exactly(cuda, H, S, D, bits, ak, av, L, B, layout, seed):
     """Every quantization axis pair (quantizer_func.py:41-49) on drawn geometries, with
-    head-split sections and per-head levels: the generic row kernels run the oracle's
-    stage order, so the stream bytes, metadata and decompressed KV are bit-exact (a
-    default pair on an MFMA geometry is held to the configuration bars instead)."""
+    head-split sections and per-head levels: the generic row kernels (fwht="rows") run the
+    oracle's stage order, so the stream bytes, metadata and decompressed KV are bit-exact."""
+    _axes_sweep(cuda, H, S, D, bits, ak, av, L, B, layout, seed, "rows")
+
+
+@pytest.mark.parametrize("H,S,D,bits,ak,av,L,B,layout,seed", AXES_SWEEP)
+def test_axes_sweep_on_the_default_kernels(cuda, H, S, D, bits, ak, av, L, B, layout, seed):
+    """The same draws on the kernels they run by themselves, held to the configuration bars."""
+    _axes_sweep(cuda, H, S, D, bits, ak, av, L, B, layout, seed, "mfma")
+
+
+def _axes_sweep(cuda, H, S, D, bits, ak, av, L, B, layout, seed, fwht):
     from kvserve_amd.engine import FusedKVCodec, check_packet
     from kvserve_amd.profiles import per_head_profile, section_profile
     from kvserve_amd.workloads import kv_blocks
@@ -170,16 +181,16 @@ def test_axes_sweep_matches_oracle_exactly(cuda, H, S, D, bits, ak, av, L, B, la
         else:
             prof.append(per_head_profile([int(v) for v in torch.randint(2, top + 1, (H,), generator=g)],
                                          [int(v) for v in torch.randint(2, top + 1, (H,), generator=g)]))
-    print(f"axes sweep {axes} H={H} S={S} D={D} bits={bits} L={L} B={B} {layout} seed={seed}", flush=True)
+    print(f"axes sweep {axes} H={H} S={S} D={D} bits={bits} L={L} B={B} {layout} {fwht} seed={seed}", flush=True)
     pools = [p.to(cuda) for p in pools]
     dev_ids = ids.to(torch.int32).to(cuda)
-    codec = FusedKVCodec(H, D, S, bits, 0xC0FEBABE, layout=layout, axes=axes)
+    codec = FusedKVCodec(H, D, S, bits, 0xC0FEBABE, layout=layout, axes=axes, fwht=fwht)
     packet = codec.compress(pools, dev_ids, prof)
     check_packet(packet)
     dst = [torch.zeros_like(p) for p in pools]
     codec.decompress(packet, dst, dev_ids)
     torch.cuda.synchronize()
-    if axes == ("channel", "token"):
+    if fwht == "mfma":
         for l in range(L):
             _check_layer(packet, l, _bits(pools[l][:, dev_ids.long()]), _bits(dst[l][:, dev_ids.long()]))
         return
