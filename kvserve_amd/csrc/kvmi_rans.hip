@@ -24,10 +24,11 @@
 // per symbol (A. D. Robison, "N-bit unsigned division via N-bit multiply-add", ARITH 2005).
 //
 // What bounds them (256 CUs; us before and after the present form, 134 M symbols of 3 bits in
-// 2048 blocks / 33.5 M of 8 bits in 512 blocks).  Encoding, 112 -> 79 / 52 -> 32: the vector
+// 2048 blocks / 14.7 M of 8 bits in 224 blocks, a part of the runtime's chunk; 33.5 M in 512 blocks
+// take 57 -> 38 and 52 -> 43).  Encoding, 112 -> 78 / 52 -> 32: the vector
 // units' issue at 8 waves a SIMD (instructions per symbol count: table fields where an
 // instruction takes them without an extract, two 32-bit products less), the latency of a step
-// at 2.  Decoding, 92 -> 76 / 45 -> 37.5: a step is two dependent LDS reads and a dozen
+// at 1.  Decoding, 92 -> 75 / 44 -> 37: a step is two dependent LDS reads and a dozen
 // dependent instructions; at 8 waves a SIMD its LDS conflicts (random table slots) and issue
 // overlap only in part.  The workgroup's LDS stays under 20 KB so that a CU holds 8 and 2048
 // blocks run as one round; the words, header, counts, states and first refill are requested

@@ -1,12 +1,13 @@
 // Decode pass of the wave-tile kernels (kvmi_tile.hpp): unpack, dequantize on any axis,
 // inverse transform, scatter into the paged caches.
 //
-// Bound by its writes: long enough requests reach the rate of a device copy (32 layers x 8192
-// tokens x 8 heads of 128 channels without transform 1.34 GB in 0.22 ms), shorter ones end with
-// a partly filled last round.  Measured against the row kernels that ran these calls before:
-// 16 layers x 4080 tokens x 6 heads of 96 channels 141 -> 49 us (188 MB), 16 x 4096 x 8 of 128
-// with K per token and V per channel 173 -> 78 us, without the transform (quad kernels before)
-// 143 -> 68 us.
+// Bound by its writes in long requests, which reach the rate of a device copy (32 layers x 8192
+// tokens x 8 heads of 128 channels without transform 1.34 GB in 0.22 ms); in shorter ones by vector
+// issue (half to two thirds of the busy time), trips to memory (half of a wave's time) and a partly
+// filled last round (profiles/case_kernels.md).  Against the row kernels that ran these calls
+// before: 16 layers x 4080 tokens x 6 heads of 96 channels 141 -> 47 us (192 MB, 4.1 TB/s), 16 x
+// 4096 x 8 of 128 with K per token and V per channel 173 -> 74, without the transform (quad kernels
+// before) 143 -> 63 us (342 MB, 5.4 TB/s).
 #include "kvmi_tile.hpp"
 
 namespace kvmi {

@@ -1,12 +1,12 @@
 // Encode pass of the wave-tile kernels (kvmi_tile.hpp): gather, transform, quantize on any
 // axis, bitpack.
 //
-// Bound by VALU issue together with the short runs of the permuted stream: at 12 waves a CU
-// the rounding chain (about 10 instructions an element) is 40 % of the time and a wave waits
-// for loads another 35 %.  Measured against the row kernels that ran these calls before:
-// 16 layers x 4080 tokens x 6 heads of 96 channels 259 -> 54 us (188 MB, 3.5 TB/s), 16 x 4096
-// x 8 of 128 with K per token and V per channel 283 -> 88 us, without the transform (quad
-// kernels before) 200 -> 71 us (336 MB, 4.7 TB/s).
+// Bound by vector issue (71 % of the time its CUs are busy, conversions counted once though they
+// take two slots) and by the trips to memory behind it (a wave waits for 39 % of its time at 12
+// waves a CU); it reads and writes what it must, 150 + 40 MB of 16 layers x 4080 tokens x 6
+// heads of 96 channels at 3.3 TB/s (profiles/case_kernels.md).  Against the row kernels that ran
+// these calls before: that one 259 -> 57 us, 16 x 4096 x 8 of 128 with K per token and V per
+// channel 283 -> 87, without the transform (quad kernels before) 200 -> 74 us (343 MB, 4.6 TB/s).
 #include "kvmi_tile.hpp"
 
 namespace kvmi {

@@ -16,7 +16,8 @@ constexpr int kStatTok = 32;  // tokens of a statistics tile
 // short calls, blockIdx.z), head by head; where a wave leaves a head it adds the pairs to the
 // workgroup's LDS keys.  Bound by its reads and
 // their latency (8 waves a CU): K of 16 layers x 4080 tokens x 6 heads of 96 channels (75 MB)
-// 47 us on the row kernels, 20 here (3.8 TB/s); V of 16 x 4096 x 8 of 128 (134 MB) 72 -> 30 us.
+// 47 us on the row kernels, 19 here (92 MB with the line halves beside a head's 192 bytes, 5.0
+// TB/s); V of 16 x 4096 x 8 of 128 (134 MB) 72 -> 28 us.
 template <int D>
 __global__ __launch_bounds__(kTileThreads, D <= 80 ? 4 : D <= 128 ? 3 : 2) void tile_stats_kernel(Geo g, TileArgs a,
                                                                   const kvmi_layer_job* __restrict__ jobs) {
@@ -159,7 +160,8 @@ __global__ __launch_bounds__(kTileThreads, D <= 80 ? 4 : D <= 128 ? 3 : 2) void 
 
 // Without the transform a token's H D values are plain columns: a thread keeps 8 channels
 // and walks the tokens of the run, kPlainAhead loads in flight (K of 16 layers x 4096 tokens
-// x 8 heads of 128, 134 MB: 42 us on the quad kernels, 31 here, 4.3 TB/s).
+// x 8 heads of 128, 134 MB: 42 us on the quad kernels, 29 here, 4.7 TB/s; with the caches' rows
+// still in the last-level cache 29 and 32).
 constexpr int kPlainAhead = 4;
 __global__ __launch_bounds__(kTileThreads) void tile_plain_stats_kernel(Geo g, TileArgs a,
                                                                         const kvmi_layer_job* __restrict__ jobs) {
@@ -274,14 +276,15 @@ int slots(const Geo& g, const TileArgs& a) {
 
 constexpr int kStaticLds = 1024;                  // TileTables and the like, rounded up
 constexpr int kMaxLds = 80 * 1024 - kStaticLds;   // two workgroups a CU
-// A wave's image grows, tile by tile, until a head's run in the stream is kRunBytes long (or
-// the image kImageBytes, or a wave would be left without a super-tile).  Longer runs beat
-// more resident workgroups: 16 layers x 4096 tokens x 8 heads of 128 channels, 4 bits, K per
-// token and V per channel (encode / decode us): runs of 256 bytes, 3 workgroups a CU 101 / 81,
-// of 512 95 / 73, of 1024 and 2 workgroups 90 / 70; 6 heads of 96 channels: runs of 240 bytes
-// 61 / 62, of 480 58 / 58, of 720 53 / 48.
+// A wave's image grows, tile by tile, until a head's run in the stream is kRunBytes long, or the
+// image has more slots than a wave of decode holds (max_slots; that ends 6 heads of 96 at 480
+// bytes and 8 of 128 at 512, 4 heads of 64 go to 768), or a wave would be left without a
+// super-tile.  One tile an image against the rule, at 16 layers and 4 bits (encode / decode us):
+// 4080 tokens x 6 of 96: 240 bytes 57.9 / 50.5, 480 bytes 55.6 / 45.4; 4096 x 12 of 192: 192
+// bytes 239 / 226, 576 bytes 229 / 199; K per token and V per channel 4096 x 8 of 128: 256 bytes
+// 85.4 / 68.5, 512 bytes 82.0 / 64.3; 8192 x 4 of 64: 256 bytes 46.9 / 40.7, 768 bytes 44.4 / 34.3
+// (1024 bytes 41.4 / 37.5).
 constexpr int kRunBytes = 720;
-constexpr int kImageBytes = 9 * 1024;
 constexpr int kTileRounds = 3;  // workgroups per resident slot: 1, 2, 4 and 6 within 5 %
 // 16-byte slots of an image: 64 * kPackedRegs of kvmi_tile_dec.hip
 int max_slots(const Geo& g) { return g.D <= 128 ? 256 : 512; }
@@ -371,7 +374,7 @@ TileArgs tile_plan(const Geo& g, int32_t max_blocks, int32_t num_jobs, int occ) 
   int nt = 1;
   for (int k = 2; k <= 16 && (nt * T) * RB < kRunBytes; ++k) {
     const TileArgs b = shape(g, k);
-    if (b.runs * b.pitch > kImageBytes || slots(g, b) > max_slots(g) || lds_bytes(b) > kMaxLds ||
+    if (slots(g, b) > max_slots(g) || lds_bytes(b) > kMaxLds ||
         tiles / k < resident(b) * kTileWaves)
       break;
     nt = k;
