@@ -19,8 +19,8 @@
 // Waves do not wait for each other: a wave packs NT tiles of one part into its own LDS
 // image, one run of NT * T tokens per head (permuted order), and writes the runs in
 // 16-byte pieces; decode reads them the same way.  The only workgroup barriers are those
-// behind the table set-up.  The symbol width is a kernel argument (a uniform branch per 16
-// symbols), so one kernel per head size serves every width.
+// behind the table set-up.  4 bits has kernels of its own; the other widths share one per head
+// size, with the width a kernel argument (a uniform branch per 16 symbols).
 #pragma once
 
 #include <type_traits>
